@@ -59,10 +59,10 @@ struct SBLists {
   const int32_t* stats;         // the binning's stats
 };
 
-// Images of fewer tiles are composited with four waves per tile (one pixel per lane), each
-// of which would queue the tile's entries from the superblock lists itself; with small
-// Gaussians a superblock list holds 15-50 words per entry of a tile, and the forward then
-// costs more than the write sweep saves (cfg1: 124 -> 194 us against 93 -> 80 us).
+// Images of fewer tiles are composited with sixteen waves per tile, each of which would queue
+// the tile's entries from the superblock lists itself; with small Gaussians a superblock list
+// holds 15-50 words per entry of a tile, and already with four waves per tile the forward
+// then cost more than the write sweep saves (cfg1: 124 -> 194 us against 93 -> 80 us).
 constexpr int kDeferMinTiles = 2048;
 
 // Whether a deferred binning leaves the entry list unwritten: the image has at least

@@ -13,10 +13,10 @@
 //
 // Work decomposition: every wave owns PPT*4 rows of one 16x16 tile; lane l holds the
 // PPT pixels (l % 16, row0 + l / 16 + 4 i), i < PPT, i.e. one column, so the x offset
-// to a Gaussian is shared by the lane's pixels.  Waves are independent (no LDS, no
-// barriers).  With PPT = 4 a wave covers the whole tile (used for large images);
-// PPT = 1 uses four waves per tile for small images that would otherwise leave CUs
-// idle; the forward of mid-size images uses PPT = 2 (two waves per tile).
+// to a Gaussian is shared by the lane's pixels.  Waves are independent (no barriers).  With
+// PPT = 4 a wave covers the whole tile (used for large images); the backward of small images
+// takes PPT = 1 (four waves per tile), the forward of mid-size images PPT = 2 (two waves per
+// tile).  The forward of small images has a kernel of its own (composite_fwd_quad_kernel).
 //
 // Culling: a Gaussian is binned to every tile its square 3-sigma box touches, but its
 // "power > -10" region is an ellipse, and for about a third of the (tile, entry) pairs
@@ -367,6 +367,228 @@ __device__ inline uint64_t probe_test(const Probe& p, float x0, float x1, float 
   return __ballot(p.g >= 0 && !entry_misses_rect(p.mx, p.my, p.A, p.B, p.C, x0, x1, y0, y1));
 }
 
+// Every workgroup of a forward launch clears its slice of the caller's array after its own
+// outputs (stores and loads share one wait counter, so stores issued before the walk would
+// hold up its first loads).
+__device__ inline void clear_share(float4* __restrict__ clear, int64_t n_clear) {
+  if (clear != nullptr) {
+    const int64_t per = (n_clear + gridDim.x - 1) / gridDim.x;
+    const int64_t c0 = per * blockIdx.x, c1 = c0 + per < n_clear ? c0 + per : n_clear;
+    for (int64_t c = c0 + threadIdx.x; c < c1; c += 64) clear[c] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+}
+
+// The forward of small images (below 2048 tiles).  A tile's walk is a serial chain, and the
+// longest tile's chain is the launch's time: with one pixel per lane and four waves per tile
+// an entry cost such a wave 185 cycles (16k Gaussians, 256x256, longest tile 1144 entries:
+// 88 us) while most issue slots were empty.  Here a wave owns 4 x 4 pixels and takes four
+// entries a step: lane 4 p + e evaluates entry e of the step at pixel p, and the
+// transmittance before each entry is an exclusive product of (1 - alpha) over the pixel's
+// quad of lanes (DPP), so the chain through T is one step per four entries and sixteen
+// waves share a tile.  The rectangle test runs against the wave's own 4 x 4 pixels, which
+// drops far more entries than a 16 x 4 band does.  The survivors' records are compacted into
+// LDS a batch of 64 at a time (every lane holds one entry's whole record, loaded a batch
+// ahead), from where the four records of a step are broadcast reads, two steps at a time so
+// that their exponents overlap (16k: one step at a time 35 us, two 30).
+// Forward, four waves per tile -> this: 16k, 256x256 88 -> 28 us; 200k, 504x378 130 -> 62;
+// 50k, 640x479 102 -> 52; 2k, 96x64 49 -> 15.
+constexpr int kQuadSwap1 = 0xB1;  // quad_perm [1,0,3,2]
+constexpr int kQuadSwap2 = 0x4E;  // quad_perm [2,3,0,1]
+constexpr int kQuadPrev = 0x90;   // quad_perm [0,0,1,2]
+template <int CTRL>
+__device__ inline int quad_i(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ inline float quad_f(float v) {
+  return __int_as_float(quad_i<CTRL>(__float_as_int(v)));
+}
+__device__ inline float quad_sum(float v) {
+  v += quad_f<kQuadSwap1>(v);
+  return v + quad_f<kQuadSwap2>(v);
+}
+
+constexpr int kQuadParts = 16;  // waves (4 x 4 pixel blocks) per tile
+// Workgroups of the quad forward: blocks of 128 take eight tiles, one per XCD, so that a
+// tile's sixteen waves read its records through one L2.
+__host__ __device__ inline int quad_blocks(int TX, int TY) { return ((tile_blocks(TX, TY) + 7) & ~7) * kQuadParts; }
+
+template <bool WIN>
+__global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
+    const float4* __restrict__ rec, int num_g, const int32_t* __restrict__ gids, int64_t n_entries,
+    const int32_t* __restrict__ ranges, int W, int H, int TX, int T, const float* __restrict__ bg,
+    float* __restrict__ img, float* __restrict__ finalT, int32_t* __restrict__ ncontrib,
+    int32_t* __restrict__ tile_cost, float4* __restrict__ clear, int64_t n_clear,
+    const gs_window_t* __restrict__ win, const float* __restrict__ l1_tgt, float* __restrict__ l1_part) {
+  // a batch's surviving records: 64, seven null entries that fill the last pair of steps, and
+  // nine that the last pair's prefetch reads without using them
+  __shared__ float4 sa[80], sb[80], sc[80];
+  auto clear_slice = [&]() { clear_share(clear, n_clear); };
+  const int b = (int)(blockIdx.x >> 7) * 8 + (int)(blockIdx.x & 7), part = (int)(blockIdx.x >> 3) & 15;
+  const int tile = b < tile_blocks(TX, T / TX) ? tile_of_block(b, TX, T / TX) : -1;
+  if (tile < 0) {
+    if (l1_part != nullptr && threadIdx.x == 0) l1_part[blockIdx.x] = 0.0f;
+    clear_slice();
+    return;
+  }
+  const int lane = threadIdx.x, e = lane & 3;
+  const int tx = tile % TX, ty = tile / TX;
+  const int xl = 4 * (part & 3), yl = 4 * (part >> 2);  // the block inside the tile
+  const int X = tx * kTile + xl + ((lane >> 2) & 3), Y = ty * kTile + yl + (lane >> 4);
+  const float px = (float)(tx * kTile) + ((float)(xl + ((lane >> 2) & 3)) + 0.5f);
+  const float py = (float)(ty * kTile) + ((float)(yl + (lane >> 4)) + 0.5f);
+  const float rx0 = (float)(tx * kTile + xl) + 0.5f, rx1 = rx0 + 3.0f;
+  const float ry0 = (float)(ty * kTile + yl) + 0.5f, ry1 = ry0 + 3.0f;
+  const bool inside = X < W && Y < H;
+  // a pixel outside the image starts closed, so that it never holds the wave
+  float Tr = inside ? 1.0f : 0.0f;  // before the step; below the threshold it only shrinks
+  float Tend = 0.0f;                // a closed pixel's transmittance, at its last entry
+  float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;  // this lane's entries' share of the colour
+  int cnt = 0;
+  uint64_t open = __ballot(Tr > kTMin);
+  int start, n;
+  tile_span(ranges, tile, n_entries, num_g, start, n);
+  const int64_t thr = WIN ? win->thr : 0;
+
+  struct Row {
+    int g;
+    float4 a, b, c;
+  };
+  auto load_row = [&](int g) {
+    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    Row r{g, z, z, z};
+    if (g >= 0) {
+      r.a = rec[(int64_t)g * 3];
+      r.b = rec[(int64_t)g * 3 + 1];
+      r.c = rec[(int64_t)g * 3 + 2];
+    }
+    return r;
+  };
+  // the lane's entry of a step: its record (mx my A B | C log2(op) r g | b op threshold, with
+  // the list position in the last place)
+  struct Step {
+    float4 a, b, c;
+  };
+  auto read_step = [&](int s) { return Step{sa[s + e], sb[s + e], sc[s + e]}; };
+  auto alpha = [&](const Step& k) {
+    const float dx = px - k.a.x, dy = py - k.a.y;
+    const float q = q_of(dy, fmaf(k.a.z * dx, dx, k.b.y), k.a.w * dx, k.b.x);
+    float al = __builtin_amdgcn_exp2f(q);
+    al = al < 0.99f ? al : 0.99f;
+    return q > k.c.z ? al : 0.0f;  // rasterizer.py:212
+  };
+  // product of (1 - alpha) over the step's entries before the lane's, and over all four
+  // (every lane of the quad forms the same bits)
+  auto products = [&](float al, float& ex, float& all) {
+    const float om = 1.0f - al;
+    const float om1 = quad_f<kQuadSwap1>(om);
+    const float pr = om * om1;
+    const float pr2 = quad_f<kQuadSwap2>(pr);
+    ex = ((lane & 1) ? om1 : 1.0f) * ((lane & 2) ? pr2 : 1.0f);
+    all = pr * pr2;
+  };
+  // A pixel closes at the first entry of the step after which T is below the threshold: its T
+  // there and the entry's position in the list end the pixel.  T0, T1: before and after.
+  auto close = [&](const Step& k, float T0, float before, float T1) {
+    if (T0 > kTMin && !(T1 > kTMin)) {
+      const bool past = !(before > kTMin);  // closed at an earlier lane's entry
+      const int pos = __float_as_int(k.c.w), prev = quad_i<kQuadPrev>(pos);
+      int at = past ? prev : (e == 3 ? pos : 0x7FFFFFFF);
+      float te = past ? before : (e == 3 ? T1 : 0.0f);
+      at = min(at, quad_i<kQuadSwap1>(at));
+      at = min(at, quad_i<kQuadSwap2>(at));
+      te = fmaxf(te, quad_f<kQuadSwap1>(te));
+      te = fmaxf(te, quad_f<kQuadSwap2>(te));
+      cnt = at + 1;
+      Tend = te;
+    }
+  };
+  auto walk_pair = [&](const Step& k0, const Step& k1) {
+    const float al0 = alpha(k0), al1 = alpha(k1);
+    float ex0, all0, ex1, all1;
+    products(al0, ex0, all0);
+    products(al1, ex1, all1);
+    const float T1 = Tr * all0, b0 = Tr * ex0;
+    const float T2 = T1 * all1, b1 = T1 * ex1;
+    const float w0 = b0 > kTMin ? al0 * b0 : 0.0f;  // rasterizer.py:206
+    const float w1 = b1 > kTMin ? al1 * b1 : 0.0f;
+    c0 = fmaf(w1, k1.b.z, fmaf(w0, k0.b.z, c0));
+    c1 = fmaf(w1, k1.b.w, fmaf(w0, k0.b.w, c1));
+    c2 = fmaf(w1, k1.c.x, fmaf(w0, k0.c.x, c2));
+    const uint64_t still = __ballot(T2 > kTMin);
+    if (still != open) {
+      close(k0, Tr, b0, T1);
+      close(k1, T1, b1, T2);
+      open = still;
+    }
+    Tr = T2;
+  };
+  Ahead g_ahead = probe_gid_ahead<WIN>(gids, start, 64 + lane, n, win, thr);
+  Row row = load_row(probe_gid<WIN>(gids, start, lane, n, num_g, win, thr));
+  for (int b0 = 0; b0 < n && open != 0ull; b0 += 64) {
+    const bool keep =
+        row.g >= 0 && !entry_misses_rect(row.a.x, row.a.y, row.a.z, row.a.w, row.b.x, rx0, rx1, ry0, ry1);
+    const uint64_t m = __ballot(keep);
+    const int ns = __popcll(m);
+    // the last batch's reads are done (a wave's LDS operations complete in order)
+    if (keep) {
+      const int at = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+      sa[at] = row.a;
+      sb[at] = row.b;
+      sc[at] = make_float4(row.c.x, row.c.y, row.c.z, __int_as_float(b0 + lane));
+    }
+    if (lane < 7) {  // entries no pixel passes: exponent and threshold far apart
+      sa[ns + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      sb[ns + lane] = make_float4(0.0f, -1e30f, 0.0f, 0.0f);
+      sc[ns + lane] = make_float4(0.0f, 0.0f, 1e30f, __int_as_float(0x7FFFFFFF));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // lanes read what other lanes wrote
+    row = load_row(ahead_gid(g_ahead, num_g));
+    g_ahead = probe_gid_ahead<WIN>(gids, start, b0 + 128 + lane, n, win, thr);
+    if (ns == 0) continue;
+    // steps in pairs (their exponents overlap), two sets of registers used in turn
+    Step x0 = read_step(0), x1 = read_step(4), y0, y1;
+    for (int s = 0;;) {
+      y0 = read_step(s + 8);
+      y1 = read_step(s + 12);
+      walk_pair(x0, x1);
+      s += 8;
+      if (s >= ns || open == 0ull) break;
+      x0 = read_step(s + 8);
+      x1 = read_step(s + 12);
+      walk_pair(y0, y1);
+      s += 8;
+      if (s >= ns || open == 0ull) break;
+    }
+  }
+  const bool closed = !((open >> lane) & 1ull);
+  const float Tf = closed ? Tend : Tr;
+  c0 = quad_sum(c0);
+  c1 = quad_sum(c1);
+  c2 = quad_sum(c2);
+  float l1 = 0.0f;
+  if (inside) {
+    // lane e of the quad stores channel e; lane 3 the residuals
+    const int64_t p = (int64_t)Y * W + X;
+    if (e < 3) {
+      const float o = (e == 0 ? c0 : (e == 1 ? c1 : c2)) + Tf * bg[e];
+      img[3 * p + e] = o;
+      if (l1_tgt != nullptr) l1 = fabsf(o - l1_tgt[3 * p + e]);
+    } else {
+      if (finalT) finalT[p] = Tf;
+      // a pixel still open met every entry of the tile, culled ones included
+      if (ncontrib) ncontrib[p] = closed ? cnt : n;
+    }
+  }
+  if (l1_part != nullptr) {
+    l1 = wave_sum(l1);
+    if (lane == 0) l1_part[blockIdx.x] = l1;
+  }
+  // the launch order of gs_composite_bwd ranks the tiles by the entries their lists hold
+  if (tile_cost && part == 0 && lane == 0) tile_cost[tile] = n;
+  clear_slice();
+}
+
 // WIN: the default path's chunk windows (see probe_gid); without it the id fetch compiles
 // to the plain one.
 // SB (gs_composite_fwd_deferred): when the binning deferred the entry list
@@ -385,16 +607,7 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
     const gs_window_t* __restrict__ win, const SBLists sbl, int32_t* __restrict__ gids_out,
     const float* __restrict__ l1_tgt, float* __restrict__ l1_part) {
   constexpr int WPT = 4 / PPT;  // waves per tile
-  // Every workgroup clears its slice of the caller's array after its own outputs (stores
-  // and loads share one wait counter, so stores issued before the walk would hold up its
-  // first loads).
-  auto clear_slice = [&]() {
-    if (clear != nullptr) {
-      const int64_t per = (n_clear + gridDim.x - 1) / gridDim.x;
-      const int64_t c0 = per * blockIdx.x, c1 = c0 + per < n_clear ? c0 + per : n_clear;
-      for (int64_t c = c0 + threadIdx.x; c < c1; c += 64) clear[c] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-  };
+  auto clear_slice = [&]() { clear_share(clear, n_clear); };
   const int b = blockIdx.x / WPT, part = blockIdx.x % WPT;
   const int tile = tile_of_block(b, TX, T / TX);
   if (tile < 0) {
@@ -428,15 +641,10 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
   // Walks the survivors m of a batch (lane j's record key in gk); kpos(j) is the index in
   // the tile's list of the batch's entry j.
   auto walk = [&](uint64_t m, const int gk, auto kpos) {
-    // Survivors are walked in groups of G (G = 2 when a lane holds one pixel): the
-    // group's records are in SGPRs before it is blended and the next group's scalar
-    // loads are issued first, so their latency is covered by G entries' arithmetic
-    // (scalar loads complete out of order: waiting for one is waiting for all, so
-    // requests go out per group).  With two or four pixels per lane the arithmetic of one
-    // entry covers the load and G = 1 keeps the instruction count down; its two record
-    // registers are used in turn, with an explicit wait before each request (two-wave
-    // forward, cfg4 175 -> 155 us, cfg3 148 -> 135 us; one-wave cfg2 unchanged).
-    constexpr int G = PPT == 1 ? 2 : 1;
+    // The next survivor's record is requested before the current one is blended, into two
+    // record registers used in turn, with an explicit wait before each request (scalar loads
+    // complete out of order: waiting for one is waiting for all; two-wave forward, cfg4
+    // 175 -> 155 us, cfg3 148 -> 135 us; one-wave cfg2 unchanged).
     // one walked entry e (tile index kidx within the batch) blended into the lane's pixels
     // (two or four pixels per lane: branch-free, gated-out pixels blend alpha = 0, which
     // leaves C and T unchanged; measured faster than per-pixel branches, 226 vs 251 us
@@ -460,9 +668,7 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
         cnt[i] = act ? kk : cnt[i];
       }
     };
-    if constexpr (G == 1) {
-      // one entry at a time, the next survivor's record requested before the blend; two
-      // record registers used in turn (no copy of the prefetched record per entry)
+    {
       Rec ra = zero_rec(), rb = zero_rec();
       int ja = -1, jb = -1;
       if (m != 0ull) {
@@ -509,79 +715,6 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
           ++walked;
           blend(rb, jb);
           if (ja < 0) {
-            more = false;
-            break;
-          }
-        }
-      }
-    } else {
-      // one pixel per lane: survivors in pairs, both records requested together a pair
-      // ahead, two pairs of record registers used in turn, the exit test once per 8
-      auto take = [&](Rec* r, int* j) {
-#pragma unroll
-        for (int h = 0; h < G; ++h) {
-          j[h] = -1;
-          if (m != 0ull) {
-            j[h] = __builtin_ctzll(m);
-            m &= ~(1ull << j[h]);
-            r[h] = load_rec_key<O32>(rec, bcast_i(gk, j[h]));
-          }
-        }
-      };
-      auto blend_pair = [&](const Rec* e, const int* k) {
-#pragma unroll
-        for (int h = 0; h < G; ++h) {
-          if (k[h] < 0) break;
-          ++walked;
-          const int kk = kpos(k[h]) + 1;  // entries met so far, this one included
-          const float dx = px - e[h].mx;
-          const float Adx2l = fmaf(e[h].A * dx, dx, e[h].lop), Bdx = e[h].B * dx;
-#pragma unroll
-          for (int i = 0; i < PPT; ++i) {
-            const float q = q_of(py[i] - e[h].my, Adx2l, Bdx, e[h].C);
-            const bool act = Tr[i] > kTMin;  // rasterizer.py:206
-            cnt[i] = act ? kk : cnt[i];
-            // one pixel per lane: only the lanes that pass run the blend (the wave skips it
-            // when none does; cfg1 187 -> 180 us against the branch-free form)
-            if (act && q > e[h].thr) {  // rasterizer.py:212
-              float al = __builtin_amdgcn_exp2f(q);
-              al = al < 0.99f ? al : 0.99f;
-              const float w = al * Tr[i];
-              c0[i] = fmaf(w, e[h].r, c0[i]);
-              c1[i] = fmaf(w, e[h].g, c1[i]);
-              c2[i] = fmaf(w, e[h].b, c2[i]);
-              Tr[i] = Tr[i] - w;  // T (1 - alpha)
-            }
-          }
-        }
-      };
-      Rec ra[G], rb[G];
-      int ja[G], jb[G];
-#pragma unroll
-      for (int h = 0; h < G; ++h) ra[h] = rb[h] = zero_rec();
-      take(ra, ja);
-      bool more = ja[0] >= 0;
-      while (more) {
-        bool live = false;
-#pragma unroll
-        for (int i = 0; i < PPT; ++i) live = live || Tr[i] > kTMin;
-        if (__ballot(live) == 0ull) {
-          done = true;
-          break;
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-          take(rb, jb);
-          blend_pair(ra, ja);
-          if (jb[0] < 0) {
-            more = false;
-            break;
-          }
-          __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-          take(ra, ja);
-          blend_pair(rb, jb);
-          if (ja[0] < 0) {
             more = false;
             break;
           }
@@ -1254,10 +1387,10 @@ extern "C" int gs_window_from_list(void* stream, const int32_t* sorted_gids, int
 
 namespace {
 // Floats of the l1_out array of the fused L1 loss: the loss, then one partial sum per
-// compositing workgroup (at most four per tile cell of the launch grid).
+// compositing workgroup (at most two per tile cell of the launch grid; small images, sixteen).
 int64_t l1_out_floats(int width, int height) {
   const int TX = (width + kTile - 1) / kTile, TY = (height + kTile - 1) / kTile;
-  return 1 + 4 * (int64_t)tile_blocks(TX, TY);
+  return 1 + (pick_ppt(TX * TY) == 4 ? 2 * (int64_t)tile_blocks(TX, TY) : (int64_t)quad_blocks(TX, TY));
 }
 
 int composite_fwd_run(const char* name, void* stream, int64_t n, const float* records, const int32_t* sorted_gids,
@@ -1295,15 +1428,22 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
   } else if (pick_ppt(T) == 4) {
     if (win) { GS_FWD_LAUNCH(2, 2, true); } else { GS_FWD_LAUNCH(2, 2, false); }
   } else {
-    if (win) { GS_FWD_LAUNCH(1, 4, true); } else { GS_FWD_LAUNCH(1, 4, false); }
+    // below kDeferMinTiles the entry list is always whole
+#define GS_FWD_QUAD(WIN)                                                                                          \
+  hipLaunchKernelGGL((composite_fwd_quad_kernel<WIN>), dim3(quad_blocks(TX, TY)), dim3(64), 0, s,                 \
+                     (const float4*)records, (int)n, sorted_gids, n_entries, ranges, width, height, TX, T,        \
+                     background, image, final_T, n_contrib, tile_order, (float4*)clear_records, n4_clear, window, \
+                     l1_target, l1_part)
+    if (win) GS_FWD_QUAD(true); else GS_FWD_QUAD(false);
+#undef GS_FWD_QUAD
   }
 #undef GS_FWD_LAUNCH
 #undef GS_FWD_LAUNCH1
 #undef GS_FWD_LAUNCH2
   GS_LAUNCH_CHECK("composite_fwd_kernel");
   if (tile_order || l1_out) {
-    const int wpt = pick_ppt(T) == 4 ? (T >= kFwdOneWaveTiles ? 1 : 2) : 4;
-    hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, tile_order, T, l1_part, nblk * wpt,
+    const int nparts = pick_ppt(T) == 4 ? nblk * (T >= kFwdOneWaveTiles ? 1 : 2) : quad_blocks(TX, TY);
+    hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, tile_order, T, l1_part, nparts,
                        (int64_t)width * height * 3, l1_out);
     GS_LAUNCH_CHECK("tile_order_kernel");
   }
