@@ -89,7 +89,8 @@ const char* gs_last_error(void);
  * gs_composite_bwd_l1.  13: gs_bin and gs_bin_deferred take the chunk window (the binning
  * builds it; gs_window_from_bins stays for lists binned without it).  14: gs_composite_bwd
  * and gs_composite_bwd_l1 take a gs_clear_list_t; gs_preprocess_bwd and
- * gs_preprocess_bwd_w2c take zeroed. */
+ * gs_preprocess_bwd_w2c take zeroed.  Added since, with every call of 14 as it was:
+ * gs_composite_segments_size, gs_composite_fwd_seg, gs_composite_bwd_seg. */
 int gs_abi_version(void);
 
 /* Projection + covariance + SH colour for every Gaussian.
@@ -320,6 +321,32 @@ int gs_composite_bwd_l1(void* stream, int64_t n, const float* records, const int
                         const float* final_T, const int32_t* n_contrib, const int32_t* tile_order,
                         float* grad_records, float* grad_background, int accumulate, const gs_window_t* window,
                         const gs_clear_list_t* clear);
+
+/* Compositing with the lists cut into segments, so that the backward walks a tile's entries
+ * in several waves at once (a tile's walk is a serial chain; the longest one was most
+ * launches' time).  Replaces the same reference code as gs_composite_fwd and gs_composite_bwd.
+ *
+ * gs_composite_segments_size: bytes of the segments array (16-byte aligned) that the forward
+ *   writes and the backward of the same render reads.
+ * gs_composite_fwd_seg: gs_composite_fwd (stats and bin_workspace NULL; capacity = the list's
+ *   length) or gs_composite_fwd_deferred (both given), with segments in tile_order's place;
+ *   l1_target and l1_out (NULL, or both as in gs_composite_fwd_deferred_l1) fuse the L1 loss.
+ * gs_composite_bwd_seg: gs_composite_bwd, or with image, l1_target and l1_cot
+ *   gs_composite_bwd_l1 (grad_image may then be NULL), with that segments array in
+ *   tile_order's place.  The gradients are the same sums: the transmittance and the colour
+ *   behind a segment's last entry come from the forward instead of the entries behind it. */
+size_t gs_composite_segments_size(int width, int height);
+int gs_composite_fwd_seg(void* stream, int64_t n, const float* records, int32_t* sorted_gids, int64_t capacity,
+                         const int32_t* ranges, const int32_t* stats, const void* bin_workspace,
+                         size_t bin_workspace_bytes, int width, int height, const float* background, float* image,
+                         float* final_T, int32_t* n_contrib, void* segments, float* clear_records,
+                         const gs_window_t* window, const float* l1_target, float* l1_out);
+int gs_composite_bwd_seg(void* stream, int64_t n, const float* records, const int32_t* sorted_gids,
+                         int64_t n_entries, const int32_t* ranges, int width, int height, const float* background,
+                         const float* grad_image, const float* image, const float* l1_target, const float* l1_cot,
+                         const float* final_T, const int32_t* n_contrib, const void* segments, float* grad_records,
+                         float* grad_background, int accumulate, const gs_window_t* window,
+                         const gs_clear_list_t* clear);
 
 /* Vector-Jacobian product of gs_preprocess_fwd's compositing records with respect to
  * the five Gaussian parameter arrays (JAX autodiff of project_gaussians, eval_sh,

@@ -81,6 +81,13 @@ __device__ inline float wave_sum(float v) {
   return bcast(x, 63);
 }
 
+// Largest of the 64 lanes' values, in every lane.
+__device__ inline int wave_max(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return bcast_i(v, 0);
+}
+
 // The image cotangent the backward reads per pixel: dL/dimage (gimg), and/or the VJP of the
 // L1 loss fused into the compositing (losses.py:4-8) when tgt is set: sign(image - target)
 // times (dL/dloss) / count, sign(0) = 0, formed as the separate loss VJP forms it.
@@ -378,6 +385,60 @@ __device__ inline void clear_share(float4* __restrict__ clear, int64_t n_clear) 
   }
 }
 
+constexpr int kQuadTiles = 2048;  // images below are composited by composite_fwd_quad_kernel
+
+// Segments of a tile's list.  The backward walks a tile's entries back to front, a serial
+// chain like the forward's, and the longest tile's chain was most launches' time (2170 tiles
+// of 274 entries on average: the one of 1046 took 283 us while the work of all would fill the
+// GPU for 50).  The forward therefore cuts every list into segments, 1024/u of u entries, then
+// 512/u of 2u and 512/u of 4u (4096 in all; log2 u = segment_shift), and leaves for each segment it
+// completes, per pixel, the transmittance after it and the colour blended in it.  The backward
+// then walks all segments at once: a segment starts from its own end's transmittance, and the
+// colour behind it is the background's share plus the later segments' colours, summed from
+// the back, so neither is recovered through the entries behind it.
+// Backward, whole lists -> segments: 300k Gaussians at 979x546 283 -> 95 us, 200k at 504x378
+// 217 -> 75, 50k at 640x479 170 -> 66, 2k at 96x64 90 -> 22, 2.1M at 1280x720 284 -> 197 (which
+// zeroes 500 MB besides); the order of the items instead of the tiles' 4.8 -> 10 us, the slots
+// add 5-8 us to the forward.
+// Slot j of a tile (256 pixels, row by row): (T after segment j, colour r g b of segment j).
+// A pixel's slots are written for every segment it enters, except where its wave never leaves
+// segment 0 (there the final T and the background say it all).
+// The backward's work items are pieces: the segments of a coarser unit, the smallest of u, 2u,
+// .. 512 at which the pieces of all tiles fit the launch's grid (segment_grid; every coarser
+// unit's ends are ends of segments of u, and at 512 a tile has at most four).
+struct Segments {
+  int32_t* items;   // [0] = number of pieces, [1] = log2 of their unit, then tile * 32 + piece, longest first
+  int32_t* met;     // per tile, the entries met by each of the forward's waves
+  float4* slots;    // [T][segment_count(u)][256]; NULL: the forward leaves none
+  int lu;           // log2(u)
+};
+// From kFwdOneWaveTiles tiles on, one wave per tile fills the GPU several times over, and the
+// slots' traffic and the pieces' set-up cost more than they balance (8160 tiles, the longest
+// of 781 entries: backward 247 -> 255 us, its order 8 -> 13 us): no segments there.
+constexpr int kFwdOneWaveTiles = 6 * 1024;
+// Units: 64 entries where tiles are few (200k Gaussians, 504x378: 128 91 us, 64 75), 128 where
+// they fill the GPU sooner and a piece's set-up has to be earned back (300k, 979x546: 64 99 us,
+// 128 95, 256 121).
+__host__ __device__ inline int segment_shift(int T) { return T < kQuadTiles ? 6 : 7; }  // log2(u)
+__host__ __device__ inline int segment_count(int lu) { return 2048 >> lu; }
+__host__ __device__ inline int segment_start(int j, int lu) {
+  const int n0 = 1024 >> lu, n1 = n0 + (n0 >> 1);
+  return j <= n0 ? j << lu : (j <= n1 ? 1024 + ((j - n0) << (lu + 1)) : 2048 + ((j - n1) << (lu + 2)));
+}
+// segments that hold the first k entries (k <= 4096)
+__host__ __device__ inline int segments_within(int k, int lu) {
+  const int n0 = 1024 >> lu, n1 = n0 + (n0 >> 1);
+  const int up = (1 << lu) - 1, up1 = (2 << lu) - 1, up2 = (4 << lu) - 1;
+  return k <= 1024 ? (k + up) >> lu : (k <= 2048 ? n0 + ((k - 1024 + up1) >> (lu + 1)) : n1 + ((k - 2048 + up2) >> (lu + 2)));
+}
+// Most pieces a launch takes.  Workgroups past the pieces' number exit at once, but each
+// still costs its dispatch (3600 tiles with room for 16 pieces each, 57,600 workgroups of which
+// 10,000 had work: 232 us against 203).
+__host__ __device__ inline int segment_grid(int T) {
+  const int all = T * segment_count(segment_shift(T)), some = 4 * T + 2048;
+  return all < some ? all : some;
+}
+
 // The forward of small images (below 2048 tiles).  A tile's walk is a serial chain, and the
 // longest tile's chain is the launch's time: with one pixel per lane and four waves per tile
 // an entry cost such a wave 185 cycles (16k Gaussians, 256x256, longest tile 1144 entries:
@@ -419,7 +480,8 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
     const int32_t* __restrict__ ranges, int W, int H, int TX, int T, const float* __restrict__ bg,
     float* __restrict__ img, float* __restrict__ finalT, int32_t* __restrict__ ncontrib,
     int32_t* __restrict__ tile_cost, float4* __restrict__ clear, int64_t n_clear,
-    const gs_window_t* __restrict__ win, const float* __restrict__ l1_tgt, float* __restrict__ l1_part) {
+    const gs_window_t* __restrict__ win, const float* __restrict__ l1_tgt, float* __restrict__ l1_part,
+    const Segments sg) {
   // a batch's surviving records: 64, seven null entries that fill the last pair of steps, and
   // nine that the last pair's prefetch reads without using them
   __shared__ float4 sa[80], sb[80], sc[80];
@@ -443,8 +505,9 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
   // a pixel outside the image starts closed, so that it never holds the wave
   float Tr = inside ? 1.0f : 0.0f;  // before the step; below the threshold it only shrinks
   float Tend = 0.0f;                // a closed pixel's transmittance, at its last entry
-  float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;  // this lane's entries' share of the colour
-  int cnt = 0;
+  float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;  // this lane's entries' share of the segment's colour
+  float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;  // the pixel's colour of the segments before it
+  int cnt = 0, seg = 0, seg_end = 1 << sg.lu;
   uint64_t open = __ballot(Tr > kTMin);
   int start, n;
   tile_span(ranges, tile, n_entries, num_g, start, n);
@@ -525,7 +588,25 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
   };
   Ahead g_ahead = probe_gid_ahead<WIN>(gids, start, 64 + lane, n, win, thr);
   Row row = load_row(probe_gid<WIN>(gids, start, lane, n, num_g, win, thr));
+  // the segment's colour summed over the quad and, with the transmittance, left for the backward
+  auto end_segment = [&](float Tnow) {
+    c0 = quad_sum(c0);
+    c1 = quad_sum(c1);
+    c2 = quad_sum(c2);
+    if (sg.slots != nullptr && e == 0)
+      sg.slots[((int64_t)tile * segment_count(sg.lu) + seg) * 256 + (yl + (lane >> 4)) * kTile + xl +
+               ((lane >> 2) & 3)] = make_float4(Tnow, c0, c1, c2);
+  };
   for (int b0 = 0; b0 < n && open != 0ull; b0 += 64) {
+    if (b0 == seg_end) {
+      end_segment(Tr);
+      s0 += c0;
+      s1 += c1;
+      s2 += c2;
+      c0 = c1 = c2 = 0.0f;
+      ++seg;
+      seg_end = segment_start(seg + 1, sg.lu);
+    }
     const bool keep =
         row.g >= 0 && !entry_misses_rect(row.a.x, row.a.y, row.a.z, row.a.w, row.b.x, rx0, rx1, ry0, ry1);
     const uint64_t m = __ballot(keep);
@@ -563,9 +644,17 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
   }
   const bool closed = !((open >> lane) & 1ull);
   const float Tf = closed ? Tend : Tr;
-  c0 = quad_sum(c0);
-  c1 = quad_sum(c1);
-  c2 = quad_sum(c2);
+  if (seg > 0) {
+    end_segment(Tf);
+    c0 += s0;
+    c1 += s1;
+    c2 += s2;
+  } else {
+    c0 = quad_sum(c0);
+    c1 = quad_sum(c1);
+    c2 = quad_sum(c2);
+  }
+  const int nc = closed ? cnt : n;  // a pixel still open met every entry of the tile, culled ones included
   float l1 = 0.0f;
   if (inside) {
     // lane e of the quad stores channel e; lane 3 the residuals
@@ -576,9 +665,12 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
       if (l1_tgt != nullptr) l1 = fabsf(o - l1_tgt[3 * p + e]);
     } else {
       if (finalT) finalT[p] = Tf;
-      // a pixel still open met every entry of the tile, culled ones included
-      if (ncontrib) ncontrib[p] = closed ? cnt : n;
+      if (ncontrib) ncontrib[p] = nc;
     }
+  }
+  if (sg.met != nullptr) {
+    const int k = wave_max(inside ? nc : 0);
+    if (lane == 0) sg.met[tile * kQuadParts + part] = k;
   }
   if (l1_part != nullptr) {
     l1 = wave_sum(l1);
@@ -605,8 +697,10 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
     float* __restrict__ img, float* __restrict__ finalT, int32_t* __restrict__ ncontrib,
     int32_t* __restrict__ tile_cost, float4* __restrict__ clear, int64_t n_clear,
     const gs_window_t* __restrict__ win, const SBLists sbl, int32_t* __restrict__ gids_out,
-    const float* __restrict__ l1_tgt, float* __restrict__ l1_part) {
+    const float* __restrict__ l1_tgt, float* __restrict__ l1_part, const Segments sg) {
   constexpr int WPT = 4 / PPT;  // waves per tile
+  constexpr bool SEGS = PPT < 4;  // one wave per tile: no segments (kFwdOneWaveTiles)
+  __shared__ float s_col[SEGS ? 3 * PPT : 1][64];  // the colour of the segments before the current one (read from segment 1 on)
   auto clear_slice = [&]() { clear_share(clear, n_clear); };
   const int b = blockIdx.x / WPT, part = blockIdx.x % WPT;
   const int tile = tile_of_block(b, TX, T / TX);
@@ -638,6 +732,37 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
 
   bool done = false;
   int walked = 0;
+  // The segment's colour and the transmittance after it, left for the backward; the colour
+  // then moves to LDS (touched only here: in registers it would be live through the walk).
+  int seg = 0, seg_end = 1 << sg.lu;
+  auto end_segment = [&]() {
+    if constexpr (SEGS)
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+      if (sg.slots != nullptr)
+        sg.slots[((int64_t)tile * segment_count(sg.lu) + seg) * 256 + (part * 4 * PPT + (lane >> 4) + 4 * i) * kTile +
+                 (lane & 15)] = make_float4(Tr[i], c0[i], c1[i], c2[i]);
+      if (seg > 0) {
+        c0[i] += s_col[3 * i][lane];
+        c1[i] += s_col[3 * i + 1][lane];
+        c2[i] += s_col[3 * i + 2][lane];
+      }
+    }
+  };
+  auto at_batch = [&](int b0) {
+    if constexpr (!SEGS) return;
+    if (b0 != seg_end) return;
+    end_segment();
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+      s_col[SEGS ? 3 * i : 0][lane] = c0[i];
+      s_col[SEGS ? 3 * i + 1 : 0][lane] = c1[i];
+      s_col[SEGS ? 3 * i + 2 : 0][lane] = c2[i];
+      c0[i] = c1[i] = c2[i] = 0.0f;
+    }
+    ++seg;
+    seg_end = segment_start(seg + 1, sg.lu);
+  };
   // Walks the survivors m of a batch (lane j's record key in gk); kpos(j) is the index in
   // the tile's list of the batch's entry j.
   auto walk = [&](uint64_t m, const int gk, auto kpos) {
@@ -734,6 +859,7 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
     Ahead g_ahead = probe_gid_ahead<WIN>(gids, start, 64 + lane, n, win, thr);
     Probe pr = probe_load(rec, probe_gid<WIN>(gids, start, lane, n, num_g, win, thr));
     for (int b0 = 0; b0 < n && !done; b0 += 64) {
+      at_batch(b0);
       const int gk = rec_key<O32>(pr.g);  // the lane's record key (read where the lane survives)
       const uint64_t m = probe_test(pr, rx0, rx1, ry0, ry1);
       pr = probe_load(rec, ahead_gid(g_ahead, num_g));
@@ -819,6 +945,7 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
       WordAhead a_ahead = word_ahead(64 + lane);
       Probe pr = probe_load(rec, take_gid(word_ahead(lane), lane));
       for (int b0 = 0; b0 < n && !done; b0 += 64) {
+        at_batch(b0);
         const int gk = rec_key<O32>(pr.g);
         const uint64_t m = probe_test(pr, rx0, rx1, ry0, ry1);
         pr = probe_load(rec, take_gid(a_ahead, b0 + 64 + lane));
@@ -828,6 +955,8 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
       }
     }
   }
+  if (SEGS && seg > 0) end_segment();
+  int kmax = 0;
   const float bg0 = bg[0], bg1 = bg[1], bg2 = bg[2];
   // the L1 loss against l1_tgt (losses.py:4-8): the lane's sum of |image - target| over its
   // pixels' channels, reduced over the wave into the workgroup's partial
@@ -843,7 +972,9 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
       img[3 * p + 2] = o2;
       if (finalT) finalT[p] = Tr[i];
       // a pixel still open met every entry of the tile, culled ones included
-      if (ncontrib) ncontrib[p] = Tr[i] > kTMin ? n : cnt[i];
+      const int nc = Tr[i] > kTMin ? n : cnt[i];
+      if (ncontrib) ncontrib[p] = nc;
+      kmax = max(kmax, nc);
       if (l1_tgt != nullptr)
         l1 += (fabsf(o0 - l1_tgt[3 * p]) + fabsf(o1 - l1_tgt[3 * p + 1])) + fabsf(o2 - l1_tgt[3 * p + 2]);
     }
@@ -851,6 +982,10 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
   if (l1_part != nullptr) {
     l1 = wave_sum(l1);
     if (lane == 0) l1_part[blockIdx.x] = l1;
+  }
+  if (SEGS && sg.met != nullptr) {
+    kmax = wave_max(kmax);
+    if (lane == 0) sg.met[tile * WPT + part] = kmax;
   }
   // walk length of the tile (first wave of the tile): the backward's cost estimate
   // (two waves per tile: each stores its own length in one 16-bit half, the order takes
@@ -871,16 +1006,16 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
 // an rcp and a product.  Both NOCAP changes keep the loop-carried state in place (a body
 // chosen per entry between two versions made the compiler copy that state at every entry).
 // More registers live than the 64-VGPR build allows.
-template <int PPT, bool WIN, bool NOCAP, bool O32>
+template <int PPT, bool WIN, bool NOCAP, bool O32, bool SEG>
 __device__ __forceinline__ void composite_bwd_body(
     const float4* __restrict__ rec, int num_g, const int32_t* __restrict__ gids, int64_t n_entries,
     const int32_t* __restrict__ ranges, int W, int H, int TX, int T, const float* __restrict__ bg,
     const ImageCot gc, const float* __restrict__ finalT, const int32_t* __restrict__ ncontrib,
-    float* __restrict__ grec, const int32_t* __restrict__ order, const gs_window_t* __restrict__ win) {
-  constexpr int WPT = 4 / PPT;
-  const int b = blockIdx.x / WPT, part = blockIdx.x % WPT;
-  const int tile = order ? (b < T ? order[b] : -1) : tile_of_block(b, TX, T / TX);
-  if (tile < 0 || tile >= T) return;
+    float* __restrict__ grec, const gs_window_t* __restrict__ win, const Segments sg, int tile, int piece, int part) {
+  // the entries to walk: a piece of the list, or all of it
+  const int lp = SEG ? sg.items[1] : 0;
+  const int lo = SEG ? segment_start(piece, lp) : 0, hi = SEG ? segment_start(piece + 1, lp) : kMaxTileEntries;
+  const int last = SEG ? segments_within(hi, sg.lu) - 1 : 0;  // the piece's last segment
   const int lane = threadIdx.x;
   const int tx = tile % TX, ty = tile / TX;
   const int X = tx * kTile + (lane & 15);
@@ -899,18 +1034,33 @@ __device__ __forceinline__ void composite_bwd_body(
     const int yl = part * 4 * PPT + (lane >> 4) + 4 * i;
     py[i] = (float)(ty * kTile) + ((float)yl + 0.5f);
     Tr[i] = 1.0f;  // NOCAP: the reciprocal 1/T (see the body)
-    g0[i] = g1[i] = g2[i] = 0.0f;
+    g0[i] = g1[i] = g2[i] = Rg[i] = 0.0f;
     kp[i] = 0;
     const int Y = Y0 + 4 * i;
     if (X < W && Y < H) {
       const int64_t p = (int64_t)Y * W + X;
-      Tr[i] = NOCAP ? 1.0f / fmaxf(finalT[p], 1e-30f) : finalT[p];  // finite for T = 0
-      const int k = ncontrib[p];
-      kp[i] = k < 0 ? 0 : (k > n ? n : k);  // entries beyond the tile's list never load
+      float Tq = finalT[p];
+      int k = ncontrib[p];
+      k = k < 0 ? 0 : (k > n ? n : k);  // entries beyond the tile's list never load
+      kp[i] = min(k, hi);
       image_cot(gc, l1sc, p, g0[i], g1[i], g2[i]);
+      // colour behind the last entry is the background
+      Rg[i] = fmaf(bg2, g2[i], fmaf(bg1, g1[i], bg0 * g0[i]));
+      if (SEG && k > hi) {
+        // behind the piece's last entry: the background and the later segments' colours,
+        // farthest first, over the transmittance there
+        const float4* slot =
+            sg.slots + (int64_t)tile * segment_count(sg.lu) * 256 + (part * 4 * PPT + (lane >> 4) + 4 * i) * kTile + (lane & 15);
+        float R = Tq * Rg[i];
+        for (int j = segments_within(k, sg.lu) - 1; j > last; --j) {
+          const float4 d = slot[j * 256];
+          R += fmaf(d.w, g2[i], fmaf(d.z, g1[i], d.y * g0[i]));
+        }
+        Tq = slot[last * 256].x;
+        Rg[i] = R / Tq;  // the pixel went on: Tq > 1e-4
+      }
+      Tr[i] = NOCAP ? 1.0f / fmaxf(Tq, 1e-30f) : Tq;  // finite for T = 0
     }
-    // colour behind the last entry is the background
-    Rg[i] = fmaf(bg2, g2[i], fmaf(bg1, g1[i], bg0 * g0[i]));
     kmax = max(kmax, kp[i]);
     kmin = min(kmin, X < W && Y0 + 4 * i < H ? kp[i] : 0);
   }
@@ -924,7 +1074,7 @@ __device__ __forceinline__ void composite_bwd_body(
   kmax = bcast_i(kmax, 0);
   kmin = bcast_i(kmin, 0);
 
-  // entries kmax-1 .. 0 in batches of 64 from the top; surviving entries walked from
+  // entries kmax-1 .. lo (a multiple of 64) in batches of 64 from the top; surviving entries walked from
   // the highest down, ids from the testing lane, records by scalar loads, prefetched
   const float rx0 = (float)(tx * kTile) + 0.5f, rx1 = rx0 + (float)(kTile - 1);
   const float ry0 = (float)(ty * kTile + part * 4 * PPT) + 0.5f, ry1 = ry0 + (float)(4 * PPT - 1);
@@ -935,7 +1085,7 @@ __device__ __forceinline__ void composite_bwd_body(
   const int64_t thr = WIN ? win->thr : 0;
   Ahead g_ahead = probe_gid_ahead<WIN>(gids, start, btop - 64 + lane, kmax, win, thr);
   Probe p_next = probe_load(rec, probe_gid<WIN>(gids, start, btop + lane, kmax, num_g, win, thr));
-  for (int b0 = btop; b0 >= 0; b0 -= 64) {
+  for (int b0 = btop; b0 >= lo; b0 -= 64) {
     const Probe pr = p_next;
     p_next = probe_load(rec, ahead_gid(g_ahead, num_g));
     g_ahead = probe_gid_ahead<WIN>(gids, start, b0 - 128 + lane, kmax, win, thr);
@@ -1184,8 +1334,26 @@ __device__ inline void clear_list_share(const ClearList& cl, int b, int nb, int 
   const float4 *__restrict__ rec, int num_g, const int32_t *__restrict__ gids, int64_t n_entries,               \
       const int32_t *__restrict__ ranges, int W, int H, int TX, int T, const float *__restrict__ bg,            \
       const ImageCot gc, const float *__restrict__ finalT, const int32_t *__restrict__ ncontrib,               \
-      float *__restrict__ grec, const int32_t *__restrict__ order, const gs_window_t *__restrict__ win
-#define GS_BWD_ARGS rec, num_g, gids, n_entries, ranges, W, H, TX, T, bg, gc, finalT, ncontrib, grec, order, win
+      float *__restrict__ grec, const int32_t *__restrict__ order, const gs_window_t *__restrict__ win,          \
+      const Segments sg, const ClearList cl
+#define GS_BWD_ARGS rec, num_g, gids, n_entries, ranges, W, H, TX, T, bg, gc, finalT, ncontrib, grec, win, sg
+
+// What a workgroup walks: with segments (SEG), an item, none past their number; without, a
+// whole tile, from the launch order or the fixed one.
+template <bool SEG>
+__device__ __forceinline__ bool walk_of_block(const Segments& sg, const int32_t* __restrict__ order, int TX, int T,
+                                              int b, int& tile, int& piece) {
+  if (SEG) {
+    if (b >= sg.items[0]) return false;
+    const int v = sg.items[2 + b];
+    tile = v >> 5;
+    piece = v & 31;
+  } else {
+    tile = order ? (b < T ? order[b] : -1) : tile_of_block(b, TX, T / TX);
+    piece = 0;
+  }
+  return tile >= 0 && tile < T;
+}
 
 // The backward's two builds.  One pixel per lane (images below 2048 tiles, four waves per
 // tile): 64 VGPRs, 8 waves per SIMD, the general body only (the no-cap path's per-entry test
@@ -1202,16 +1370,19 @@ __device__ inline void clear_list_share(const ClearList& cl, int b, int nb, int 
 // windows, as the forward read them.
 // Each workgroup zeroes its share of the clear list after its walk (stores issued before it
 // would hold up its first loads: loads and stores share one wait counter).
-template <int PPT, bool WIN, bool O32>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void composite_bwd_kernel(GS_BWD_PARAMS,
-                                                                                                     const ClearList cl) {
-  composite_bwd_body<PPT, WIN, false, O32>(GS_BWD_ARGS);
+template <bool WIN, bool O32, bool SEG>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void composite_bwd_kernel(GS_BWD_PARAMS) {
+  int tile, piece;
+  if (walk_of_block<SEG>(sg, order, TX, T, blockIdx.x >> 2, tile, piece))
+    composite_bwd_body<1, WIN, false, O32, SEG>(GS_BWD_ARGS, tile, piece, blockIdx.x & 3);
   clear_list_share(cl, blockIdx.x, gridDim.x, threadIdx.x);
 }
-template <bool WIN, bool O32>
+template <bool WIN, bool O32, bool SEG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 5))) void composite_bwd_wide_kernel(
-    GS_BWD_PARAMS, const ClearList cl) {
-  composite_bwd_body<4, WIN, true, O32>(GS_BWD_ARGS);
+    GS_BWD_PARAMS) {
+  int tile, piece;
+  if (walk_of_block<SEG>(sg, order, TX, T, blockIdx.x, tile, piece))
+    composite_bwd_body<4, WIN, true, O32, SEG>(GS_BWD_ARGS, tile, piece, 0);
   clear_list_share(cl, blockIdx.x, gridDim.x, threadIdx.x);
 }
 #undef GS_BWD_PARAMS
@@ -1270,26 +1441,12 @@ __global__ __launch_bounds__(256) void background_grad_kernel(int64_t npix, int 
 constexpr int kOrderMaxTiles = 65536;
 constexpr int kOrderBuckets = 1024;  // walk lengths <= 4096 -> buckets <= 512
 
-// The same workgroup finishes the fused L1 loss: loss = (sum of the forward's per-workgroup
-// partials) / count, the partials added in a fixed order (no atomics: the same value on
+// The fused L1 loss: loss = (sum of the forward's per-workgroup partials) / count, the partials
+// added in a fixed order by the one workgroup of 1024 threads (no atomics: the same value on
 // every run).
-__global__ __launch_bounds__(1024) void tile_order_kernel(int32_t* __restrict__ order, int T,
-                                                          const float* __restrict__ l1_part, int nparts,
-                                                          int64_t count, float* __restrict__ l1_loss) {
-  __shared__ uint16_t bucket[kOrderMaxTiles];
-  __shared__ int start[kOrderBuckets];
-  __shared__ int wsum[16];
-  __shared__ float fsum[16];
+__device__ inline void finish_l1(const float* __restrict__ l1_part, int nparts, int64_t count,
+                                 float* __restrict__ l1_loss, float* fsum) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  // the workgroup is latency-bound: the first 8 walk lengths and the partials of each round
-  // of 8 are requested together, before anything waits for them
-  const bool ord = order != nullptr && T <= kOrderMaxTiles;
-  uint32_t w0[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int t = tid + 1024 * k;
-    w0[k] = ord && t < T ? (uint32_t)order[t] : 0u;
-  }
   if (l1_part != nullptr) {
     float a = 0.0f;
     for (int i0 = 0; i0 < nparts; i0 += 8 * 1024) {
@@ -1311,6 +1468,26 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(int32_t* __restrict__ 
       l1_loss[0] = t / (float)count;  // jnp.mean: the sum over the count
     }
   }
+}
+
+__global__ __launch_bounds__(1024) void tile_order_kernel(int32_t* __restrict__ order, int T,
+                                                          const float* __restrict__ l1_part, int nparts,
+                                                          int64_t count, float* __restrict__ l1_loss) {
+  __shared__ uint16_t bucket[kOrderMaxTiles];
+  __shared__ int start[kOrderBuckets];
+  __shared__ int wsum[16];
+  __shared__ float fsum[16];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  // the workgroup is latency-bound: the first 8 walk lengths and the partials of each round
+  // of 8 are requested together, before anything waits for them
+  const bool ord = order != nullptr && T <= kOrderMaxTiles;
+  uint32_t w0[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int t = tid + 1024 * k;
+    w0[k] = ord && t < T ? (uint32_t)order[t] : 0u;
+  }
+  finish_l1(l1_part, nparts, count, l1_loss, fsum);
   if (order == nullptr) return;
   if (T > kOrderMaxTiles) {
     for (int t = tid; t < T; t += 1024) order[t] = t;
@@ -1346,17 +1523,131 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(int32_t* __restrict__ 
   for (int t = tid; t < T; t += 1024) order[atomicAdd(&start[bucket[t]], 1)] = t;
 }
 
+// The backward's items: the pieces of every tile's list that some pixel reached, the longest
+// first by classes (4, 2 and 1 units, then quarters of a unit), and the fused L1 loss.  One
+// workgroup, so its instructions count: a tile's pieces are counted in closed form, and the
+// classes' places come from one scan of packed counts (a histogram by LDS atomics, most of
+// whose additions meet in a few buckets, took 12-16 us at 2170-3600 tiles).
+__global__ __launch_bounds__(1024) void segment_items_kernel(const Segments sg, int T, int parts, int grid,
+                                                             const float* __restrict__ l1_part, int nparts,
+                                                             int64_t count, float* __restrict__ l1_loss) {
+  constexpr int kPer = (kFwdOneWaveTiles + 1023) / 1024;  // T < kFwdOneWaveTiles
+  __shared__ uint64_t w0[16], w1[16];
+  __shared__ float fsum[16];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  int k[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int t = tid + 1024 * i;
+    k[i] = 0;
+    if (t >= T) continue;
+    if (parts == kQuadParts) {
+      const int4* p = reinterpret_cast<const int4*>(sg.met + (int64_t)t * kQuadParts);
+      const int4 a = p[0], b = p[1], c = p[2], d = p[3];
+      k[i] = max(max(max(max(a.x, a.y), max(a.z, a.w)), max(max(b.x, b.y), max(b.z, b.w))),
+                 max(max(max(c.x, c.y), max(c.z, c.w)), max(max(d.x, d.y), max(d.z, d.w))));
+    } else {
+      k[i] = max(sg.met[2 * t], sg.met[2 * t + 1]);  // two waves per tile
+    }
+    k[i] = min(k[i], kMaxTileEntries);
+  }
+  finish_l1(l1_part, nparts, count, l1_loss, fsum);
+  // the pieces at u, 2u and 4u, 21 bits each
+  uint64_t a = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i)
+    a += (uint64_t)segments_within(k[i], sg.lu) | (uint64_t)segments_within(k[i], sg.lu + 1) << 21 |
+         (uint64_t)segments_within(k[i], sg.lu + 2) << 42;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor((unsigned long long)a, o, 64);
+  if (lane == 0) w0[wid] = a;
+  __syncthreads();
+  a = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) a += w0[w];
+  __syncthreads();
+  int lp = sg.lu;
+  for (; lp < 9; ++lp, a >>= 21)
+    if (lp < sg.lu + 3 && (int)(a & 0x1FFFFF) <= grid) break;
+  // a tile's pieces: n4 of four units (entries 2048 on), n2 of two (1024 on), n1 of one, and a
+  // rest; f(class, number, first piece)
+  const int c0 = 1024 >> lp, c1 = c0 + (c0 >> 1);
+  auto pieces = [&](int n, auto f) {
+    const int n1 = min(n, 1024) >> lp, n2 = (min(max(n, 1024), 2048) - 1024) >> (lp + 1),
+              n4 = (max(n, 2048) - 2048) >> (lp + 2);
+    const int next = n > 2048 ? c1 + n4 : (n > 1024 ? c0 + n2 : n1);
+    const int rest = n - segment_start(next, lp);
+    if (n4 > 0) f(0, n4, c1);
+    if (n2 > 0) f(1, n2, c0);
+    if (n1 > 0) f(2, n1, 0);
+    if (rest > 0) f(rest >> (lp + 1) ? 1 : (rest >> lp ? 2 : 6 - (rest << 2 >> lp)), 1, next);
+  };
+  // places: 16 bits per class (a grid is below 2^16), four classes a word
+  uint64_t q0 = 0, q1 = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i)
+    pieces(k[i], [&](int c, int num, int) {
+      if (c < 4) q0 += (uint64_t)num << (16 * c);
+      else q1 += (uint64_t)num << (16 * (c - 4));
+    });
+  uint64_t x0 = q0, x1 = q1;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t y0 = __shfl_up((unsigned long long)x0, o, 64), y1 = __shfl_up((unsigned long long)x1, o, 64);
+    if (lane >= o) {
+      x0 += y0;
+      x1 += y1;
+    }
+  }
+  if (lane == 63) {
+    w0[wid] = x0;
+    w1[wid] = x1;
+  }
+  __syncthreads();
+  uint64_t t0 = 0, t1 = 0, p0 = x0 - q0, p1 = x1 - q1;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    if (w < wid) {
+      p0 += w0[w];
+      p1 += w1[w];
+    }
+    t0 += w0[w];
+    t1 += w1[w];
+  }
+  int base = 0;  // the classes one after another
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const int sh = 16 * (c & 3);
+    if (c < 4) p0 += (uint64_t)base << sh;
+    else p1 += (uint64_t)base << sh;
+    base += (int)((c < 4 ? t0 >> sh : t1 >> sh) & 0xFFFF);
+  }
+  if (tid == 0) {
+    sg.items[0] = base;
+    sg.items[1] = lp;
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i)
+    pieces(k[i], [&](int c, int num, int first) {
+      const int sh = 16 * (c & 3);
+      int32_t* out = sg.items + 2 + (int)((c < 4 ? p0 >> sh : p1 >> sh) & 0xFFFF);
+      if (c < 4) p0 += (uint64_t)num << sh;
+      else p1 += (uint64_t)num << sh;
+      for (int j = 0; j < num; ++j) out[j] = (tid + 1024 * i) * 32 + first + j;
+    });
+}
+
 // Record byte offsets (gid * 48) fit the 32-bit offset register of scalar loads.
 inline bool rec_offsets_fit(int64_t n) { return n * (int64_t)(kRec * 4) <= (int64_t)0xFFFFFFFF - 64; }
 
 // Large images have enough tiles to fill the GPU with one wave per tile.
-inline int pick_ppt(int T) { return T >= 2048 ? 4 : 1; }
+inline int pick_ppt(int T) { return T >= kQuadTiles ? 4 : 1; }
+constexpr int kSegWideTiles = 512;
 // Tiles from which the forward gives a tile one wave (four pixels per lane); below that (and
 // from 2048 tiles) two waves of eight rows each: at 3600 tiles a launch holds 3-4 waves per
 // SIMD, and halving the work units evens them out (cfg4 forward 189 -> 176 us) where at
-// 8160 tiles the duplicated per-entry work costs more than it balances (227 -> 255 us).
-constexpr int kFwdOneWaveTiles = 6 * 1024;
-
+// 8160 tiles the duplicated per-entry work costs more than it balances (227 -> 255 us):
+// kFwdOneWaveTiles.
 }  // namespace
 }  // namespace gs
 
@@ -1386,6 +1677,27 @@ extern "C" int gs_window_from_list(void* stream, const int32_t* sorted_gids, int
 }
 
 namespace {
+// A segments buffer: the items, the waves' met counts, the slots; from kFwdOneWaveTiles tiles
+// on, where lists have no segments, the tile order.
+int64_t segments_layout(int T, int64_t* met, int64_t* slots) {
+  if (T >= kFwdOneWaveTiles) return (int64_t)T * 4;
+  auto up = [](int64_t b) { return (b + 255) & ~(int64_t)255; };
+  *met = up(4 * (2 + (int64_t)segment_grid(T)));
+  *slots = *met + up((int64_t)T * (T < kQuadTiles ? kQuadParts : 2) * 4);
+  return *slots + (int64_t)T * segment_count(segment_shift(T)) * 256 * (int64_t)sizeof(float4);
+}
+Segments segments_of(void* p, int T) {
+  Segments sg{nullptr, nullptr, nullptr, segment_shift(T)};
+  if (p != nullptr) {
+    int64_t met, slots;
+    segments_layout(T, &met, &slots);
+    sg.items = (int32_t*)p;
+    sg.met = (int32_t*)((char*)p + met);
+    sg.slots = (float4*)((char*)p + slots);
+  }
+  return sg;
+}
+
 // Floats of the l1_out array of the fused L1 loss: the loss, then one partial sum per
 // compositing workgroup (at most two per tile cell of the launch grid; small images, sixteen).
 int64_t l1_out_floats(int width, int height) {
@@ -1397,7 +1709,7 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
                       int64_t n_entries, const int32_t* ranges, int width, int height, const float* background,
                       float* image, float* final_T, int32_t* n_contrib, int32_t* tile_order, float* clear_records,
                       const gs_window_t* window, const SBLists* sbl, int32_t* gids_out,
-                      const float* l1_target = nullptr, float* l1_out = nullptr) {
+                      const float* l1_target = nullptr, float* l1_out = nullptr, void* segments = nullptr) {
   GS_REQUIRE(n >= 0 && n < ((int64_t)1 << 31), "%s: n out of range", name);
   GS_REQUIRE(n_entries >= 0, "%s: n_entries must be >= 0", name);
   GS_REQUIRE(width > 0 && height > 0, "%s: bad image size %dx%d", name, width, height);
@@ -1413,11 +1725,17 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
   GS_REQUIRE((l1_target == nullptr) == (l1_out == nullptr), "%s: l1_target and l1_out go together", name);
   float* l1_part = l1_out ? l1_out + 1 : nullptr;
   const SBLists none{};
+  GS_REQUIRE(((uintptr_t)segments & 15) == 0, "%s: segments must be 16-byte aligned", name);
+  if (T >= kFwdOneWaveTiles && segments != nullptr) {
+    tile_order = (int32_t*)segments;
+    segments = nullptr;
+  }
+  const Segments sg = segments_of(segments, T);
 #define GS_FWD_LAUNCH2(PPT, WPT, WIN, O32, SB)                                                                  \
   hipLaunchKernelGGL((composite_fwd_kernel<PPT, WIN, O32, SB>), dim3(nblk * (WPT)), dim3(64), 0, s,             \
                      (const float4*)records, (int)n, sorted_gids, n_entries, ranges, width, height, TX, T,        \
                      background, image, final_T, n_contrib, tile_order, (float4*)clear_records, n4_clear, window, \
-                     SB ? *sbl : none, gids_out, l1_target, l1_part)
+                     SB ? *sbl : none, gids_out, l1_target, l1_part, sg)
 #define GS_FWD_LAUNCH1(PPT, WPT, WIN, O32) \
   if (sbl) GS_FWD_LAUNCH2(PPT, WPT, WIN, O32, true); else GS_FWD_LAUNCH2(PPT, WPT, WIN, O32, false)
 #define GS_FWD_LAUNCH(PPT, WPT, WIN) \
@@ -1433,7 +1751,7 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
   hipLaunchKernelGGL((composite_fwd_quad_kernel<WIN>), dim3(quad_blocks(TX, TY)), dim3(64), 0, s,                 \
                      (const float4*)records, (int)n, sorted_gids, n_entries, ranges, width, height, TX, T,        \
                      background, image, final_T, n_contrib, tile_order, (float4*)clear_records, n4_clear, window, \
-                     l1_target, l1_part)
+                     l1_target, l1_part, sg)
     if (win) GS_FWD_QUAD(true); else GS_FWD_QUAD(false);
 #undef GS_FWD_QUAD
   }
@@ -1441,7 +1759,13 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
 #undef GS_FWD_LAUNCH1
 #undef GS_FWD_LAUNCH2
   GS_LAUNCH_CHECK("composite_fwd_kernel");
-  if (tile_order || l1_out) {
+  if (segments) {
+    const int parts = pick_ppt(T) == 4 ? 2 : kQuadParts;
+    const int nparts = pick_ppt(T) == 4 ? nblk * parts : quad_blocks(TX, TY);
+    hipLaunchKernelGGL(segment_items_kernel, dim3(1), dim3(1024), 0, s, sg, T, parts, segment_grid(T), l1_part, nparts,
+                       (int64_t)width * height * 3, l1_out);
+    GS_LAUNCH_CHECK("segment_items_kernel");
+  } else if (tile_order || l1_out) {
     const int nparts = pick_ppt(T) == 4 ? nblk * (T >= kFwdOneWaveTiles ? 1 : 2) : quad_blocks(TX, TY);
     hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, tile_order, T, l1_part, nparts,
                        (int64_t)width * height * 3, l1_out);
@@ -1501,7 +1825,7 @@ int composite_bwd_run(const char* name, void* stream, int64_t n, const float* re
                       int64_t n_entries, const int32_t* ranges, int width, int height, const float* background,
                       const ImageCot& gc, const float* final_T, const int32_t* n_contrib,
                       const int32_t* tile_order, float* grad_records, float* grad_background, int accumulate,
-                      const gs_window_t* window, const gs_clear_list_t* clear) {
+                      const gs_window_t* window, const gs_clear_list_t* clear, const void* segments = nullptr) {
   GS_REQUIRE(n >= 0 && n < ((int64_t)1 << 31), "%s: n out of range", name);
   ClearList cl{};
   if (clear != nullptr) {
@@ -1533,29 +1857,33 @@ int composite_bwd_run(const char* name, void* stream, int64_t n, const float* re
   }
   const int TX = (width + kTile - 1) / kTile, TY = (height + kTile - 1) / kTile;
   const int T = TX * TY;
-  const int nblk = tile_blocks(TX, TY);
+  GS_REQUIRE(((uintptr_t)segments & 15) == 0, "%s: segments must be 16-byte aligned", name);
+  if (T >= kFwdOneWaveTiles && segments != nullptr) {
+    tile_order = (const int32_t*)segments;
+    segments = nullptr;
+  }
+  const Segments sg = segments_of(const_cast<void*>(segments), T);
+  const int nblk = segments ? segment_grid(T) : tile_blocks(TX, TY);
 #define GS_BWD_LAUNCH(KERNEL, WPT)                                                                                  \
   hipLaunchKernelGGL(KERNEL, dim3(nblk * (WPT)), dim3(64), 0, s, (const float4*)records, (int)n, sorted_gids, n_entries, \
                      ranges, width, height, TX, T, background, gc, final_T, n_contrib, grad_records,                   \
-                     tile_order, window, cl)
+                     tile_order, window, sg, cl)
   const bool win = window != nullptr, o32 = rec_offsets_fit(n);
-  if (pick_ppt(T) == 4) {
-    if (o32) {
-      if (win) GS_BWD_LAUNCH((composite_bwd_wide_kernel<true, true>), 1);
-      else GS_BWD_LAUNCH((composite_bwd_wide_kernel<false, true>), 1);
-    } else {
-      if (win) GS_BWD_LAUNCH((composite_bwd_wide_kernel<true, false>), 1);
-      else GS_BWD_LAUNCH((composite_bwd_wide_kernel<false, false>), 1);
-    }
-  } else {
-    if (o32) {
-      if (win) GS_BWD_LAUNCH((composite_bwd_kernel<1, true, true>), 4);
-      else GS_BWD_LAUNCH((composite_bwd_kernel<1, false, true>), 4);
-    } else {
-      if (win) GS_BWD_LAUNCH((composite_bwd_kernel<1, true, false>), 4);
-      else GS_BWD_LAUNCH((composite_bwd_kernel<1, false, false>), 4);
-    }
-  }
+  // A piece is short: from 512 tiles on one wave of four pixels per lane walks it, the fewest
+  // instructions per entry (1200 tiles: 66 us against 84 with four waves of one pixel per lane);
+  // below, those four waves (24 tiles: 22 us against 40).
+  const bool wide = segments ? T >= kSegWideTiles : pick_ppt(T) == 4;
+#define GS_BWD_LAUNCH1(WIN, O32, SEG)                                                                                \
+  if (wide) GS_BWD_LAUNCH((composite_bwd_wide_kernel<WIN, O32, SEG>), 1);                                            \
+  else GS_BWD_LAUNCH((composite_bwd_kernel<WIN, O32, SEG>), 4)
+#define GS_BWD_LAUNCH2(SEG)                                                                                          \
+  if (win && o32) { GS_BWD_LAUNCH1(true, true, SEG); }                                                               \
+  else if (o32) { GS_BWD_LAUNCH1(false, true, SEG); }                                                                \
+  else if (win) { GS_BWD_LAUNCH1(true, false, SEG); }                                                                \
+  else { GS_BWD_LAUNCH1(false, false, SEG); }
+  if (segments) { GS_BWD_LAUNCH2(true) } else { GS_BWD_LAUNCH2(false) }
+#undef GS_BWD_LAUNCH2
+#undef GS_BWD_LAUNCH1
 #undef GS_BWD_LAUNCH
   GS_LAUNCH_CHECK("composite_bwd_kernel");
   return GS_OK;
@@ -1587,4 +1915,44 @@ extern "C" int gs_composite_bwd_l1(void* stream, int64_t n, const float* records
   return composite_bwd_run("gs_composite_bwd_l1", stream, n, records, sorted_gids, n_entries, ranges, width,
                            height, background, gc, final_T, n_contrib, tile_order, grad_records, grad_background,
                            accumulate, window, clear);
+}
+
+extern "C" size_t gs_composite_segments_size(int width, int height) {
+  if (width <= 0 || height <= 0) return 0;
+  int64_t met, slots;
+  return (size_t)segments_layout(((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile), &met, &slots);
+}
+
+extern "C" int gs_composite_fwd_seg(void* stream, int64_t n, const float* records, int32_t* sorted_gids,
+                                    int64_t capacity, const int32_t* ranges, const int32_t* stats,
+                                    const void* bin_workspace, size_t bin_workspace_bytes, int width, int height,
+                                    const float* background, float* image, float* final_T, int32_t* n_contrib,
+                                    void* segments, float* clear_records, const gs_window_t* window,
+                                    const float* l1_target, float* l1_out) {
+  GS_REQUIRE(segments != nullptr, "gs_composite_fwd_seg: NULL segments");
+  GS_REQUIRE((stats == nullptr) == (bin_workspace == nullptr), "gs_composite_fwd_seg: stats and workspace go together");
+  SBLists sbl;
+  if (stats != nullptr) {
+    GS_REQUIRE(capacity > 0, "gs_composite_fwd_seg: capacity must be > 0 (got %lld)", (long long)capacity);
+    GS_REQUIRE(n == 0 || sorted_gids != nullptr, "gs_composite_fwd_seg: NULL argument");
+    const int rc = superblock_lists(n, width, height, capacity, bin_workspace, bin_workspace_bytes, stats, &sbl);
+    if (rc != GS_OK) return rc;
+  }
+  return composite_fwd_run("gs_composite_fwd_seg", stream, n, records, sorted_gids, capacity, ranges, width, height,
+                           background, image, final_T, n_contrib, nullptr, clear_records, window,
+                           stats ? &sbl : nullptr, sorted_gids, l1_target, l1_out, segments);
+}
+
+extern "C" int gs_composite_bwd_seg(void* stream, int64_t n, const float* records, const int32_t* sorted_gids,
+                                    int64_t n_entries, const int32_t* ranges, int width, int height,
+                                    const float* background, const float* grad_image, const float* image,
+                                    const float* l1_target, const float* l1_cot, const float* final_T,
+                                    const int32_t* n_contrib, const void* segments, float* grad_records,
+                                    float* grad_background, int accumulate, const gs_window_t* window,
+                                    const gs_clear_list_t* clear) {
+  GS_REQUIRE(segments != nullptr, "gs_composite_bwd_seg: NULL segments");
+  const ImageCot gc{grad_image, image, l1_target, l1_cot};
+  return composite_bwd_run("gs_composite_bwd_seg", stream, n, records, sorted_gids, n_entries, ranges, width, height,
+                           background, gc, final_T, n_contrib, nullptr, grad_records, grad_background, accumulate,
+                           window, clear, segments);
 }

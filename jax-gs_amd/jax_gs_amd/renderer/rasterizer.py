@@ -151,13 +151,45 @@ def composite_records(means2D, cov2D, opacities, colors) -> torch.Tensor:
     return rec
 
 
+def new_segments(H: int, W: int, dev) -> torch.Tensor:
+    """Storage for the segments that a compositing forward leaves to its backward."""
+    return torch.empty((_lib.lib().gs_composite_segments_size(int(W), int(H)),), dtype=torch.uint8, device=dev)
+
+
+def _check_bins(bins: BinResult, records, sorted_gids, ranges) -> None:
+    if sorted_gids is not bins["sorted_gids"] or ranges is not bins["ranges"] or records.shape[0] != bins["n"]:
+        raise ValueError("composite: bins must be the deferred binning of these entries and records")
+
+
+def _composite_segments(records, sorted_gids, ranges, H, W, background, image, fT, nc, segments, clear_records, window,
+                        bins, l1_target):
+    """composite() with segments (gs_composite_fwd_seg)."""
+    dev = records.device
+    stats = ws = tgt = l1_out = None
+    nb, capacity = 0, sorted_gids.shape[0]
+    if bins is not None and bins["deferred"]:
+        _check_bins(bins, records, sorted_gids, ranges)
+        stats, ws, capacity = bins["stats"], bins["workspace"], bins["capacity"]
+        nb = ws.shape[0]
+    if l1_target is not None:
+        tgt = check_f32("l1_target", l1_target, (H, W, 3), dev)
+        l1_out = torch.empty((_lib.lib().gs_composite_l1_out_size(int(W), int(H)),), dtype=torch.float32, device=dev)
+    _lib.call("gs_composite_fwd_seg", _lib.stream_handle(dev), records.shape[0], _lib.ptr(records),
+              _lib.ptr(sorted_gids), capacity, _lib.ptr(ranges), _lib.ptr(stats), _lib.ptr(ws), nb, int(W), int(H),
+              _lib.ptr(background), _lib.ptr(image), _lib.ptr(fT), _lib.ptr(nc), _lib.ptr(segments),
+              _lib.ptr(clear_records), _lib.ptr(window), _lib.ptr(tgt), _lib.ptr(l1_out))
+    return (image, fT, nc, None) if l1_out is None else (image, fT, nc, None, l1_out[0])
+
+
 def composite(records: torch.Tensor, sorted_gids: torch.Tensor, ranges: torch.Tensor, H: int, W: int,
               background: torch.Tensor, residuals: bool = True, clear_records: torch.Tensor | None = None,
               window: torch.Tensor | None = None, bins: BinResult | None = None,
-              l1_target: torch.Tensor | None = None):
+              l1_target: torch.Tensor | None = None, segments: torch.Tensor | None = None):
     """Front-to-back compositing; returns (image [H,W,3], final_T [H,W], n_contrib [H,W],
     tile_order [T]), the last three the backward's residuals (None unless residuals):
     tile_order lists the tiles longest walk first, the backward's launch order.
+    segments (new_segments(H, W)) takes its place (None is returned for it): the forward
+    leaves each list's segments there, which gs_composite_bwd_seg walks side by side.
     clear_records ([n, GS_REC_STRIDE] float32), when given, is set to zero by the same launch
     (for a backward that accumulates into it).  window None reads each tile's own entries
     (rasterizer_tpu.py:90-97); a window (window_from_list, bin_gaussians(window=True))
@@ -173,10 +205,12 @@ def composite(records: torch.Tensor, sorted_gids: torch.Tensor, ranges: torch.Te
     image = torch.empty((H, W, 3), dtype=torch.float32, device=dev)
     fT = torch.empty((H, W), dtype=torch.float32, device=dev) if residuals else None
     nc = torch.empty((H, W), dtype=torch.int32, device=dev) if residuals else None
+    if segments is not None:
+        return _composite_segments(records, sorted_gids, ranges, H, W, background, image, fT, nc, segments,
+                                   clear_records, window, bins, l1_target)
     order = torch.empty((T,), dtype=torch.int32, device=dev) if residuals else None
     if bins is not None and bins["deferred"]:
-        if sorted_gids is not bins["sorted_gids"] or ranges is not bins["ranges"] or records.shape[0] != bins["n"]:
-            raise ValueError("composite: bins must be the deferred binning of these entries and records")
+        _check_bins(bins, records, sorted_gids, ranges)
         ws = bins["workspace"]
         args = (_lib.stream_handle(dev), records.shape[0], _lib.ptr(records), _lib.ptr(sorted_gids), bins["capacity"],
                 _lib.ptr(ranges), _lib.ptr(bins["stats"]), _lib.ptr(ws), ws.shape[0], int(W), int(H),
@@ -209,24 +243,25 @@ class _RenderTiles(torch.autograd.Function):
     def forward(ctx, means2D, cov2D, opacities, colors, bg, gids, ranges, win, static):
         H, W = static
         rec = composite_records(means2D, cov2D, opacities, colors)
-        image, fT, nc, order = composite(rec, gids, ranges, H, W, bg, residuals=True, window=win)
+        segs = new_segments(H, W, rec.device) if any(ctx.needs_input_grad[:5]) else None
+        image, fT, nc, _ = composite(rec, gids, ranges, H, W, bg, residuals=True, window=win, segments=segs)
         ctx.static = static
-        ctx.save_for_backward(cov2D, opacities, bg, rec, gids, ranges, win, fT, nc, order)
+        ctx.save_for_backward(cov2D, opacities, bg, rec, gids, ranges, win, fT, nc, segs)
         return image
 
     @staticmethod
     def backward(ctx, g_image):
         H, W = ctx.static
-        cov2D, opacities, bg, rec, gids, ranges, win, fT, nc, order = ctx.saved_tensors
+        cov2D, opacities, bg, rec, gids, ranges, win, fT, nc, segs = ctx.saved_tensors
         dev = rec.device
         n = rec.shape[0]
         s = _lib.stream_handle(dev)
         g_image = g_image.contiguous()
         grec = torch.empty((n, _lib.GS_REC_STRIDE), dtype=torch.float32, device=dev)
         gbg = torch.empty((3,), dtype=torch.float32, device=dev) if ctx.needs_input_grad[4] else None
-        _lib.call("gs_composite_bwd", s, n, _lib.ptr(rec), _lib.ptr(gids), gids.shape[0], _lib.ptr(ranges), int(W),
-                  int(H), _lib.ptr(bg), _lib.ptr(g_image), _lib.ptr(fT), _lib.ptr(nc), _lib.ptr(order),
-                  _lib.ptr(grec), _lib.ptr(gbg), 0, _lib.ptr(win), None)
+        _lib.call("gs_composite_bwd_seg", s, n, _lib.ptr(rec), _lib.ptr(gids), gids.shape[0], _lib.ptr(ranges),
+                  int(W), int(H), _lib.ptr(bg), _lib.ptr(g_image), None, None, None, _lib.ptr(fT), _lib.ptr(nc),
+                  _lib.ptr(segs), _lib.ptr(grec), _lib.ptr(gbg), 0, _lib.ptr(win), None)
         gm = torch.empty((n, 2), dtype=torch.float32, device=dev)
         gc = torch.empty((n, 2, 2), dtype=torch.float32, device=dev)
         go = torch.empty((n, 1), dtype=torch.float32, device=dev)

@@ -6,7 +6,7 @@ The reference differentiates render with JAX autodiff; here a
 ``torch.autograd.Function`` plays the role of a ``jax.custom_vjp``: its forward runs
 the preprocessing, binning and compositing kernels and keeps the per-Gaussian
 records, the sorted entry list, the tile ranges, per-pixel (final T, entry count)
-and the backward's tile order as residuals; its backward runs the compositing VJP and the preprocessing VJP and
+and the lists' segments as residuals; its backward runs the compositing VJP and the preprocessing VJP and
 returns cotangents of the five Gaussian arrays (equal to JAX autodiff of the
 reference forward, with its tie conventions), of the background, and of the camera's
 W2C when it requires grad (through the camera-space means, W_rot and the view
@@ -30,12 +30,12 @@ from ..core.camera import Camera
 from ..core.gaussians import Gaussians
 from ._buffers import as_mask, background_tensor, check_f32, num_tiles
 from .projection import preprocess
-from .rasterizer import bin_gaussians, check_capacity, composite
+from .rasterizer import bin_gaussians, check_capacity, composite, new_segments
 
 
 def _render_forward(ctx, means, scales, quats, opac, sh, w2c, bg, mask, static, target=None):
     """The forward of _Render and _RenderL1: (image, radii, valid, stats[, loss])."""
-    W, H, fx, fy, cx, cy, sh_degree, capacity, tpu = static
+    W, H, fx, fy, cx, cy, sh_degree, capacity, tpu, grad = static
     g = Gaussians(means, scales, quats, opac, sh)
     cam = Camera(W, H, fx, fy, cx, cy, w2c, None)
     pre = preprocess(g, cam, mask=mask, sh_degree=sh_degree, records=True, projected=False)
@@ -45,17 +45,19 @@ def _render_forward(ctx, means, scales, quats, opac, sh, w2c, bg, mask, static, 
     # compositing launch (its waves are arithmetic-bound: the stores are free)
     n = means.shape[0]
     grec = (torch.empty((n, _lib.GS_REC_STRIDE), dtype=torch.float32, device=means.device)
-            if any(ctx.needs_input_grad[:5]) else None)
+            if grad and any(ctx.needs_input_grad[:5]) else None)
     win = b["window"]
-    out = composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg, residuals=True, clear_records=grec,
-                    window=win, bins=b, l1_target=target)
-    image, fT, nc, order = out[:4]
+    # the lists' segments, which the backward walks side by side
+    segs = new_segments(H, W, means.device) if grad and any(ctx.needs_input_grad) else None
+    out = composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg, residuals=segs is not None,
+                    clear_records=grec, window=win, bins=b, l1_target=target, segments=segs)
+    image, fT, nc = out[:3]
     ctx.static = static
     ctx.grec_fresh = grec is not None
     # radii, valid and stats carry no gradient: no zero cotangents for them
     ctx.set_materialize_grads(False)
     ctx.save_for_backward(means, scales, quats, opac, sh, w2c, bg, pre["records"], b["sorted_gids"], b["ranges"],
-                          fT, nc, order, grec, win, image if target is not None else None, target)
+                          fT, nc, segs, grec, win, image if target is not None else None, target)
     radii = pre["radii"]
     valid = pre["valid"].view(torch.bool)  # the kernel writes 0/1 bytes
     stats = b["stats"]
@@ -65,10 +67,10 @@ def _render_forward(ctx, means, scales, quats, opac, sh, w2c, bg, mask, static, 
 
 def _render_backward(ctx, g_image, g_loss=None):
     """Cotangents of (means, scales, quats, opacities, sh, W2C, background)."""
-    W, H, fx, fy, cx, cy, sh_degree, _, _ = ctx.static
+    W, H, fx, fy, cx, cy, sh_degree = ctx.static[:7]
     if g_image is None and g_loss is None:
         return (None,) * 7
-    (means, scales, quats, opac, sh, w2c, bg, rec, gids, ranges, fT, nc, order, grec, win, image,
+    (means, scales, quats, opac, sh, w2c, bg, rec, gids, ranges, fT, nc, segs, grec, win, image,
      target) = ctx.saved_tensors
     dev = means.device
     n = means.shape[0]
@@ -91,15 +93,13 @@ def _render_backward(ctx, g_image, g_loss=None):
     go = torch.empty_like(opac)
     gsh = torch.empty_like(sh)
     cl = _lib.clear_list(gm, gs_, gq, go, gsh)
-    head = (s, n, _lib.ptr(rec), _lib.ptr(gids), gids.shape[0], _lib.ptr(ranges), int(W), int(H), _lib.ptr(bg))
-    tail = (_lib.ptr(fT), _lib.ptr(nc), _lib.ptr(order), _lib.ptr(grec), _lib.ptr(gbg), accumulate, _lib.ptr(win),
-            ctypes.byref(cl))
-    if g_loss is not None:
-        # the fused L1 loss: its VJP is formed per pixel inside the compositing VJP
-        gl = g_loss.to(device=dev, dtype=torch.float32).contiguous()
-        _lib.call("gs_composite_bwd_l1", *head, _lib.ptr(gi), _lib.ptr(image), _lib.ptr(target), _lib.ptr(gl), *tail)
-    else:
-        _lib.call("gs_composite_bwd", *head, _lib.ptr(gi), *tail)
+    # the fused L1 loss: its VJP is formed per pixel inside the compositing VJP
+    fused = g_loss is not None
+    gl = g_loss.to(device=dev, dtype=torch.float32).contiguous() if fused else None
+    _lib.call("gs_composite_bwd_seg", s, n, _lib.ptr(rec), _lib.ptr(gids), gids.shape[0], _lib.ptr(ranges), int(W),
+              int(H), _lib.ptr(bg), _lib.ptr(gi), _lib.ptr(image if fused else None),
+              _lib.ptr(target if fused else None), _lib.ptr(gl), _lib.ptr(fT), _lib.ptr(nc), _lib.ptr(segs),
+              _lib.ptr(grec), _lib.ptr(gbg), accumulate, _lib.ptr(win), ctypes.byref(cl))
     args = (s, n, sh.shape[1], int(sh_degree), _lib.ptr(means), _lib.ptr(scales), _lib.ptr(quats), _lib.ptr(opac),
             _lib.ptr(sh), _lib.ptr(w2c), int(W), int(H), float(fx), float(fy), float(cx), float(cy), _lib.ptr(grec),
             _lib.ptr(gm), _lib.ptr(gs_), _lib.ptr(gq), _lib.ptr(go), _lib.ptr(gsh))
@@ -149,7 +149,7 @@ def _prepare(gaussians: Gaussians, camera: Camera, background, fast_tpu_rasteriz
     m = as_mask(mask, n, dev)
     cap = check_capacity(capacity, n)
     static = (int(camera.W), int(camera.H), float(camera.fx), float(camera.fy), float(camera.cx), float(camera.cy),
-              int(sh_degree), cap, bool(fast_tpu_rasterizer))
+              int(sh_degree), cap, bool(fast_tpu_rasterizer), torch.is_grad_enabled())
     return (means, gaussians.scales.contiguous(), gaussians.quaternions.contiguous(),
             gaussians.opacities.contiguous(), gaussians.sh_coeffs.contiguous(), w2c, bg, m), static
 

@@ -97,7 +97,7 @@ def _train_step_autograd(state, target_image, camera, optimizer, fast_tpu_raster
 
 def _train_step_fused(state, target_image, camera, optimizer, sh_degree, fast_tpu_rasterizer: bool = False,
                       lambda_ssim: float = 0.2):
-    from ..renderer.rasterizer import bin_gaussians, composite
+    from ..renderer.rasterizer import bin_gaussians, composite, new_segments
     from ..renderer.projection import preprocess
     from ..renderer._buffers import background_tensor
 
@@ -115,8 +115,9 @@ def _train_step_fused(state, target_image, camera, optimizer, sh_degree, fast_tp
                           window=not fast_tpu_rasterizer, deferred=True)
         bg = background_tensor(None, dev)
         grec = torch.empty((n, _lib.GS_REC_STRIDE), dtype=torch.float32, device=dev)  # cleared by the forward
-        image, fT, nc, order = composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg, residuals=True,
-                                         clear_records=grec, window=b["window"], bins=b)
+        segs = new_segments(H, W, dev)
+        image, fT, nc, _ = composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg, residuals=True,
+                                     clear_records=grec, window=b["window"], bins=b, segments=segs)
         # loss (trainer.py:18-26): one kernel for the L1 and SSIM means
         tgt = target_image.to(device=dev, dtype=torch.float32).contiguous()
         Hh, Ww, C = image.shape
@@ -131,10 +132,10 @@ def _train_step_fused(state, target_image, camera, optimizer, sh_degree, fast_tp
         gimg = torch.empty_like(image)
         _lib.call("gs_l1_ssim_bwd", s, Hh, Ww, C, _lib.ptr(image), _lib.ptr(tgt), _lib.ptr(gout), _lib.ptr(ws), nbytes,
                   _lib.ptr(gimg))
-        _lib.call("gs_composite_bwd", s, n, _lib.ptr(pre["records"]), _lib.ptr(b["sorted_gids"]),
+        _lib.call("gs_composite_bwd_seg", s, n, _lib.ptr(pre["records"]), _lib.ptr(b["sorted_gids"]),
                   b["sorted_gids"].shape[0], _lib.ptr(b["ranges"]), int(W), int(H), _lib.ptr(bg), _lib.ptr(gimg),
-                  _lib.ptr(fT), _lib.ptr(nc), _lib.ptr(order), _lib.ptr(grec), None, 1, _lib.ptr(b["window"]),
-                  None)
+                  None, None, None, _lib.ptr(fT), _lib.ptr(nc), _lib.ptr(segs), _lib.ptr(grec), None, 1,
+                  _lib.ptr(b["window"]), None)
         # preprocessing VJP + statistics + masked Adam, in place
         ost = state.opt_state
         moments = [ost.mu[f] for f in _FIELDS] + [ost.nu[f] for f in _FIELDS]
