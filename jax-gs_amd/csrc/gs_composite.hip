@@ -81,6 +81,17 @@ __device__ inline float wave_sum(float v) {
   return bcast(x, 63);
 }
 
+// Inclusive sums over the lanes (the DPP steps of wave_sum).
+__device__ inline int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+  return v;
+}
+
 // Largest of the 64 lanes' values, in every lane.
 __device__ inline int wave_max(int v) {
 #pragma unroll
@@ -871,11 +882,15 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
       // The tile's entries, in order, are the words of its superblock's list whose bit is set
       // in the tile's step masks (the binning's count sweep wrote them).  A ring of 512 word
       // positions in LDS queues the entries, so that they are probed and walked in full
-      // batches of 64 as above: fill(t) queues entries until t are queued (or the list ends),
-      // one chunk (four steps of 64 words, one mask each) at a time.  The masks of 16 chunks (64 steps) come with
-      // one vector load (lane l: step l), the next 16 a group ahead.  Entry k's id is written
-      // to gids_out[start + k] when its batch is probed (the backward's list).
-      constexpr int kRing = 512;  // live entries span < 64 + 256 (a fill overshoots by < 4 steps)
+      // batches of 64 as above: fill(t) queues entries until t are queued (or the list ends).
+      // The masks of 16 chunks (64 steps of 64 words) come with one vector load (lane l: step
+      // l), two groups ahead.  A tile whose entries are few among its superblock's words (at
+      // the edge of a dense cluster, say) has to pass over thousands of them per batch: the
+      // lanes count their steps' entries side by side and groups without any cost a ballot
+      // (four steps at a time, each tested and queued in turn, such tiles were what the launch
+      // waited for: 2.1M Gaussians at 1280x720 192 us, this 167).  Entry k's id is written to
+      // gids_out[start + k] when its batch is probed (the backward's list).
+      constexpr int kRing = 512;  // live entries span < 192 + 64 (a fill overshoots by part of a step)
       __shared__ int32_t q_lds[kRing];
       volatile int32_t* q = q_lds;  // lanes read what other lanes wrote: keep the order
       const int sx = tx / kSB, sy = ty / kSB;
@@ -885,37 +900,62 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
       c0 = c0 > sbl.n_chunks ? sbl.n_chunks : c0;
       c1 = c1 < c0 ? c0 : (c1 > sbl.n_chunks ? sbl.n_chunks : c1);
       const int64_t wbase = sbl.ranges[sbi];
-      const int nsteps = 4 * (int)(c1 - c0);
+      const int ngroups = (int)((c1 - c0 + 15) / 16);
       auto group = [&](int gi) -> uint64_t {
         const int64_t c = c0 + 16 * (int64_t)gi + (lane >> 2);
         return c < c1 ? sbl.masks[(c * 64 + u) * 4 + (lane & 3)] : 0ull;
       };
-      uint64_t mg = group(0), mg_next = group(1);
-      int sidx = 0, filled = 0;
-      // a chunk (four steps) per round: its eight mask halves are read together
+      // The current group (64 steps): lane l holds step l's mask, the number of the group's
+      // entries in the steps before it and through it, and how many of them are queued (whole
+      // steps); the next two groups' masks are on their way.
+      uint64_t mg = group(0), mg1 = group(1), mg2 = group(2);
+      int upto = wave_scan(__popcll(mg)), from = upto - __popcll(mg);
+      int gi = 0, total = bcast_i(upto, 63), taken = 0, filled = 0;
       auto fill = [&](int target) {
-        while (filled < target && sidx < nsteps) {
-          if (sidx > 0 && (sidx & 63) == 0) {
-            mg = mg_next;
-            mg_next = group((sidx >> 6) + 1);
-          }
-          uint32_t lo[4], hi[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            lo[k] = __builtin_amdgcn_readlane((uint32_t)mg, (sidx & 63) + k);
-            hi[k] = __builtin_amdgcn_readlane((uint32_t)(mg >> 32), (sidx & 63) + k);
-          }
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const uint64_t m = ((uint64_t)hi[k] << 32) | lo[k];
-            if (m != 0ull) {
-              if (__builtin_amdgcn_inverse_ballot_w64(m))
-                q[(filled + (int)__builtin_amdgcn_mbcnt_hi(hi[k], __builtin_amdgcn_mbcnt_lo(lo[k], 0u))) &
-                  (kRing - 1)] = (int32_t)(wbase + 64 * (int64_t)(sidx + k) + lane);
-              filled += __popcll(m);
+        const int goal = min(target, n);  // a list that is queued whole is not searched further
+        while (filled < goal) {
+          if (taken == total) {
+            if (++gi >= ngroups) break;
+            mg = mg1;
+            mg1 = mg2;
+            mg2 = group(gi + 2);
+            if (__ballot(mg != 0ull) == 0ull) {
+              total = 0;
+              taken = 0;
+              continue;
             }
+            const int own = __popcll(mg);
+            upto = wave_scan(own);
+            from = upto - own;
+            total = bcast_i(upto, 63);
+            taken = 0;
           }
-          sidx += 4;
+          // the steps that hold the next goal - filled entries
+          const bool sel = mg != 0ull && from >= taken && from - taken < goal - filled;
+          uint64_t steps = __ballot(sel);
+          const int end = bcast_i(upto, 63 - __builtin_clzll(steps));
+          if (__popcll(steps) <= 6) {
+            // few steps with many entries: a step at a time, a lane per word
+            for (int at = filled; steps != 0ull; steps &= steps - 1ull) {
+              const int k = __builtin_ctzll(steps);
+              const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)mg, k),
+                             hi = __builtin_amdgcn_readlane((uint32_t)(mg >> 32), k);
+              const uint64_t m = ((uint64_t)hi << 32) | lo;
+              if (__builtin_amdgcn_inverse_ballot_w64(m))
+                q[(at + (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u))) & (kRing - 1)] =
+                    (int32_t)(wbase + 64 * (int64_t)(64 * gi + k) + lane);
+              at += __popcll(m);
+            }
+          } else if (sel) {
+            // many steps with few entries each: a lane per step
+            int at = filled + from - taken;
+            const int32_t w0 = (int32_t)(wbase + 64 * (int64_t)(64 * gi + lane));
+            for (uint32_t m = (uint32_t)mg; m != 0u; m &= m - 1u) q[at++ & (kRing - 1)] = w0 + __builtin_ctz(m);
+            for (uint32_t m = (uint32_t)(mg >> 32); m != 0u; m &= m - 1u)
+              q[at++ & (kRing - 1)] = w0 + 32 + __builtin_ctz(m);
+          }
+          filled += end - taken;
+          taken = end;
         }
       };
       // entry k's word (its low half, which holds the id; loaded a batch ahead of its use),
