@@ -385,6 +385,48 @@ __device__ inline uint64_t probe_test(const Probe& p, float x0, float x1, float 
   return __ballot(p.g >= 0 && !entry_misses_rect(p.mx, p.my, p.A, p.B, p.C, x0, x1, y0, y1));
 }
 
+// What a lane of a forward wave fetches of a batch: one entry's whole record.
+struct Row {
+  int g;           // -1 past the tile's list
+  float4 a, b, c;  // mx my A B | C log2(op) r g | b op threshold no_cap
+};
+__device__ inline Row load_row(const float4* __restrict__ rec, int g) {
+  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  Row r{g, z, z, z};
+  if (g >= 0) {
+    r.a = rec[(int64_t)g * 3];
+    r.b = rec[(int64_t)g * 3 + 1];
+    r.c = rec[(int64_t)g * 3 + 2];
+  }
+  return r;
+}
+
+// Compacts a batch's survivors of the rectangle test into LDS, list positions in the records'
+// last place, followed by PAD entries that no pixel passes (exponent and threshold far
+// apart); returns their number.  A wave's LDS operations complete in order, so the reads of
+// the batch before are done.
+template <int PAD>
+__device__ inline int stage_batch(const Row& row, int b0, int lane, float rx0, float rx1, float ry0, float ry1,
+                                  float4* sa, float4* sb, float4* sc) {
+  const bool keep =
+      row.g >= 0 && !entry_misses_rect(row.a.x, row.a.y, row.a.z, row.a.w, row.b.x, rx0, rx1, ry0, ry1);
+  const uint64_t m = __ballot(keep);
+  const int ns = __popcll(m);
+  if (keep) {
+    const int at = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    sa[at] = row.a;
+    sb[at] = row.b;
+    sc[at] = make_float4(row.c.x, row.c.y, row.c.z, __int_as_float(b0 + lane));
+  }
+  if (lane < PAD) {
+    sa[ns + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    sb[ns + lane] = make_float4(0.0f, -1e30f, 0.0f, 0.0f);
+    sc[ns + lane] = make_float4(0.0f, 0.0f, 1e30f, __int_as_float(0x7FFFFFFF));
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // lanes read what other lanes wrote
+  return ns;
+}
+
 // Every workgroup of a forward launch clears its slice of the caller's array after its own
 // outputs (stores and loads share one wait counter, so stores issued before the walk would
 // hold up its first loads).
@@ -524,20 +566,6 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
   tile_span(ranges, tile, n_entries, num_g, start, n);
   const int64_t thr = WIN ? win->thr : 0;
 
-  struct Row {
-    int g;
-    float4 a, b, c;
-  };
-  auto load_row = [&](int g) {
-    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    Row r{g, z, z, z};
-    if (g >= 0) {
-      r.a = rec[(int64_t)g * 3];
-      r.b = rec[(int64_t)g * 3 + 1];
-      r.c = rec[(int64_t)g * 3 + 2];
-    }
-    return r;
-  };
   // the lane's entry of a step: its record (mx my A B | C log2(op) r g | b op threshold, with
   // the list position in the last place)
   struct Step {
@@ -598,7 +626,7 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
     Tr = T2;
   };
   Ahead g_ahead = probe_gid_ahead<WIN>(gids, start, 64 + lane, n, win, thr);
-  Row row = load_row(probe_gid<WIN>(gids, start, lane, n, num_g, win, thr));
+  Row row = load_row(rec, probe_gid<WIN>(gids, start, lane, n, num_g, win, thr));
   // the segment's colour summed over the quad and, with the transmittance, left for the backward
   auto end_segment = [&](float Tnow) {
     c0 = quad_sum(c0);
@@ -618,24 +646,8 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
       ++seg;
       seg_end = segment_start(seg + 1, sg.lu);
     }
-    const bool keep =
-        row.g >= 0 && !entry_misses_rect(row.a.x, row.a.y, row.a.z, row.a.w, row.b.x, rx0, rx1, ry0, ry1);
-    const uint64_t m = __ballot(keep);
-    const int ns = __popcll(m);
-    // the last batch's reads are done (a wave's LDS operations complete in order)
-    if (keep) {
-      const int at = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-      sa[at] = row.a;
-      sb[at] = row.b;
-      sc[at] = make_float4(row.c.x, row.c.y, row.c.z, __int_as_float(b0 + lane));
-    }
-    if (lane < 7) {  // entries no pixel passes: exponent and threshold far apart
-      sa[ns + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      sb[ns + lane] = make_float4(0.0f, -1e30f, 0.0f, 0.0f);
-      sc[ns + lane] = make_float4(0.0f, 0.0f, 1e30f, __int_as_float(0x7FFFFFFF));
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // lanes read what other lanes wrote
-    row = load_row(ahead_gid(g_ahead, num_g));
+    const int ns = stage_batch<7>(row, b0, lane, rx0, rx1, ry0, ry1, sa, sb, sc);
+    row = load_row(rec, ahead_gid(g_ahead, num_g));
     g_ahead = probe_gid_ahead<WIN>(gids, start, b0 + 128 + lane, n, win, thr);
     if (ns == 0) continue;
     // steps in pairs (their exponents overlap), two sets of registers used in turn
@@ -774,9 +786,83 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
     ++seg;
     seg_end = segment_start(seg + 1, sg.lu);
   };
-  // Walks the survivors m of a batch (lane j's record key in gk); kpos(j) is the index in
-  // the tile's list of the batch's entry j.
-  auto walk = [&](uint64_t m, const int gk, auto kpos) {
+  // Two pixels per lane (mid-size images).  There a launch waits for its longest tiles, whose
+  // waves run nearly alone on their SIMDs, so an entry's latency counts, not its instructions:
+  // with records by scalar loads an entry ahead and one dependent chain after another, a lone
+  // wave took 386 cycles an entry for 132 of issue.  The batch's survivors are staged in LDS,
+  // as in the small images' forward, and walked in pairs, all the pair's exponents first; only
+  // the transmittance links them (120 VGPRs, four waves per SIMD; capped at five waves it is
+  // slower).  300k Gaussians at 979x546 142 -> 118 us, 2.1M at 1280x720 167 -> 157, 3M in dense
+  // clusters 127 -> 112.  With four pixels per lane the same walk measures as the scalar loads
+  // do (222 us at 1920x1080), whose seven waves per SIMD hide each other's waits.
+  __shared__ float4 sa[PPT == 2 ? 72 : 1], sb[PPT == 2 ? 72 : 1], sc[PPT == 2 ? 72 : 1];
+  uint64_t open[PPT];
+#pragma unroll
+  for (int i = 0; i < PPT; ++i) open[i] = __ballot(Tr[i] > kTMin);
+  struct Ent {
+    float4 a, b, c;
+  };
+  auto read = [&](int s) { return Ent{sa[s], sb[s], sc[s]}; };
+  auto walk_pair = [&](const Ent& e0, const Ent& e1) {
+    float al0[PPT], al1[PPT], T1[PPT];
+    auto alphas = [&](const Ent& e, float* al) {
+      const float dx = px - e.a.x;
+      const float Adx2l = fmaf(e.a.z * dx, dx, e.b.y), Bdx = e.a.w * dx;
+      float q[PPT];
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) q[i] = q_of(py[i] - e.a.y, Adx2l, Bdx, e.b.x);
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) {
+        const float v = __builtin_amdgcn_exp2f(q[i]);
+        al[i] = q[i] > e.c.z ? (v < 0.99f ? v : 0.99f) : 0.0f;  // rasterizer.py:211-212
+      }
+    };
+    alphas(e0, al0);
+    alphas(e1, al1);
+    uint64_t any = 0ull, changed = 0ull, now[PPT];
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+      const float w0 = al0[i] * (Tr[i] > kTMin ? Tr[i] : 0.0f);  // rasterizer.py:206
+      T1[i] = Tr[i] - w0;
+      const float w1 = al1[i] * (T1[i] > kTMin ? T1[i] : 0.0f);
+      Tr[i] = T1[i] - w1;
+      c0[i] = fmaf(w1, e1.b.z, fmaf(w0, e0.b.z, c0[i]));
+      c1[i] = fmaf(w1, e1.b.w, fmaf(w0, e0.b.w, c1[i]));
+      c2[i] = fmaf(w1, e1.c.x, fmaf(w0, e0.c.x, c2[i]));
+      now[i] = __ballot(Tr[i] > kTMin);
+      changed |= now[i] ^ open[i];
+      any |= now[i];
+    }
+    if (changed != 0ull) {
+      // a pixel closes at the first entry after which T is below the threshold
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) {
+        if (((now[i] ^ open[i]) >> lane) & 1ull) cnt[i] = __float_as_int(T1[i] > kTMin ? e1.c.w : e0.c.w) + 1;
+        open[i] = now[i];
+      }
+      done = any == 0ull;
+    }
+  };
+  auto walk_staged = [&](int ns) __attribute__((always_inline)) {
+    if (ns == 0) return;
+    Ent x0 = read(0), x1 = read(1), y0, y1;
+    for (int s = 0;;) {
+      y0 = read(s + 2);
+      y1 = read(s + 3);
+      walk_pair(x0, x1);
+      s += 2;
+      if (s >= ns || done) break;
+      x0 = read(s + 2);
+      x1 = read(s + 3);
+      walk_pair(y0, y1);
+      s += 2;
+      if (s >= ns || done) break;
+    }
+    walked += ns;
+  };
+  // Four pixels per lane: walks the survivors m of a batch (lane j's record key in gk);
+  // kpos(j) is the index in the tile's list of the batch's entry j.
+  auto walk = [&](uint64_t m, const int gk, auto kpos) __attribute__((always_inline)) {
     // The next survivor's record is requested before the current one is blended, into two
     // record registers used in turn, with an explicit wait before each request (scalar loads
     // complete out of order: waiting for one is waiting for all; two-wave forward, cfg4
@@ -859,23 +945,40 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
     }
   };
 
+  // a batch: what a lane fetches of it, its start (the rectangle test) and its walk
+  struct Batch {
+    int gk, ns;
+    uint64_t m;
+  };
+  auto fetch = [&](int g) __attribute__((always_inline)) {
+    if constexpr (PPT == 2) return load_row(rec, g);
+    else return probe_load(rec, g);
+  };
+  auto begin = [&](const auto& f, int b0) __attribute__((always_inline)) {
+    if constexpr (PPT == 2) return Batch{0, stage_batch<1>(f, b0, lane, rx0, rx1, ry0, ry1, sa, sb, sc), 0ull};
+    else return Batch{rec_key<O32>(f.g), 0, probe_test(f, rx0, rx1, ry0, ry1)};
+  };
+  auto run = [&](const Batch& bt, int b0) __attribute__((always_inline)) {
+    if constexpr (PPT == 2) walk_staged(bt.ns);
+    else walk(bt.m, bt.gk, [&](int j) { return b0 + j; });
+  };
+
   bool deferred = false;
   if constexpr (SB) deferred = entries_deferred(sbl.stats);
   if (!deferred) {
     const int64_t thr = WIN ? win->thr : 0;
-    // The batch's probe records were requested a batch ago; the next batch's go out after
-    // the batch's test, so that the test waits for nothing requested since (loads complete
-    // in order: a wait for one waits for every earlier one), and the id two batches ahead
-    // is clamped where it is used, a batch later.
+    // The batch's records were requested a batch ago; the next batch's go out after the
+    // batch's test, so that the test waits for nothing requested since (loads complete in
+    // order: a wait for one waits for every earlier one), and the id two batches ahead is
+    // clamped where it is used, a batch later.
     Ahead g_ahead = probe_gid_ahead<WIN>(gids, start, 64 + lane, n, win, thr);
-    Probe pr = probe_load(rec, probe_gid<WIN>(gids, start, lane, n, num_g, win, thr));
+    auto fr = fetch(probe_gid<WIN>(gids, start, lane, n, num_g, win, thr));
     for (int b0 = 0; b0 < n && !done; b0 += 64) {
       at_batch(b0);
-      const int gk = rec_key<O32>(pr.g);  // the lane's record key (read where the lane survives)
-      const uint64_t m = probe_test(pr, rx0, rx1, ry0, ry1);
-      pr = probe_load(rec, ahead_gid(g_ahead, num_g));
+      const Batch bt = begin(fr, b0);
+      fr = fetch(ahead_gid(g_ahead, num_g));
       g_ahead = probe_gid_ahead<WIN>(gids, start, b0 + 128 + lane, n, win, thr);
-      walk(m, gk, [&](int j) { return b0 + j; });
+      run(bt, b0);
     }
   } else if constexpr (SB) {
     if (n > 0) {
@@ -983,15 +1086,14 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
       };
       fill(128);
       WordAhead a_ahead = word_ahead(64 + lane);
-      Probe pr = probe_load(rec, take_gid(word_ahead(lane), lane));
+      auto fr = fetch(take_gid(word_ahead(lane), lane));
       for (int b0 = 0; b0 < n && !done; b0 += 64) {
         at_batch(b0);
-        const int gk = rec_key<O32>(pr.g);
-        const uint64_t m = probe_test(pr, rx0, rx1, ry0, ry1);
-        pr = probe_load(rec, take_gid(a_ahead, b0 + 64 + lane));
+        const Batch bt = begin(fr, b0);
+        fr = fetch(take_gid(a_ahead, b0 + 64 + lane));
         fill(b0 + 192);
         a_ahead = word_ahead(b0 + 128 + lane);
-        walk(m, gk, [&](int j) { return b0 + j; });
+        run(bt, b0);
       }
     }
   }
