@@ -973,7 +973,32 @@ __device__ inline void adam_row(const AdamConsts& A, int k, float* __restrict__ 
   }
 }
 
-template <int DEG>
+// STREAM: SH parameters and moments past the memory-side cache (non-temporal 16-byte loads and
+// stores).  Arrays larger than the cache are not in it when the next step reads them, and lines
+// written with ordinary stores stay dirty there until later traffic evicts them, which the next
+// kernels pay for.  Update + the next preprocessing forward, ordinary -> non-temporal: 1M
+// Gaussians, degree 3 (576 MB of SH arrays) 299 + 89 -> 285 + 67 us; 600k 184 + 45 -> 177 + 30;
+// 300k (173 MB) 104.5 -> 98 for the update.  Arrays that fit stay in the cache from step to step:
+// 120k (69 MB) 45 -> 48.5 us, 60k 29.6 -> 31.5, so below kStreamBytes the loads are ordinary.
+constexpr int64_t kStreamBytes = (int64_t)128 << 20;
+typedef float f4nt __attribute__((ext_vector_type(4)));
+template <bool STREAM>
+__device__ inline float4 load4(const float* p, int q) {
+  if (!STREAM) return reinterpret_cast<const float4*>(p)[q];
+  const f4nt v = __builtin_nontemporal_load(reinterpret_cast<const f4nt*>(p) + q);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+template <bool STREAM>
+__device__ inline void store4(float* p, int q, const float4& v) {
+  if (!STREAM) {
+    reinterpret_cast<float4*>(p)[q] = v;
+    return;
+  }
+  const f4nt x = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(x, reinterpret_cast<f4nt*>(p) + q);
+}
+
+template <int DEG, bool STREAM>
 __global__ __launch_bounds__(64) void preprocess_bwd_adam_kernel(
     int64_t n, int K, float* __restrict__ means, float* __restrict__ scales, float* __restrict__ quats,
     float* __restrict__ opac, float* __restrict__ sh, const float* __restrict__ w2c, float fx, float fy,
@@ -1031,8 +1056,8 @@ __global__ __launch_bounds__(64) void preprocess_bwd_adam_kernel(
         const int q = v0 + 64 * u;
         if (q < nv) {
           pp[u] = reinterpret_cast<const float4*>(p)[q];
-          mm[u] = reinterpret_cast<const float4*>(mu)[q];
-          vv[u] = reinterpret_cast<const float4*>(nu)[q];
+          mm[u] = load4<STREAM>(mu, q);
+          vv[u] = load4<STREAM>(nu, q);
         }
       }
 #pragma unroll
@@ -1047,9 +1072,9 @@ __global__ __launch_bounds__(64) void preprocess_bwd_adam_kernel(
         pp[u].y = pp[u].y + adam_delta(A, 4, gr[1], mm[u].y, vv[u].y, on);
         pp[u].z = pp[u].z + adam_delta(A, 4, gr[2], mm[u].z, vv[u].z, on);
         pp[u].w = pp[u].w + adam_delta(A, 4, gr[3], mm[u].w, vv[u].w, on);
-        reinterpret_cast<float4*>(p)[q] = pp[u];
-        reinterpret_cast<float4*>(mu)[q] = mm[u];
-        reinterpret_cast<float4*>(nu)[q] = vv[u];
+        store4<STREAM>(p, q, pp[u]);
+        store4<STREAM>(mu, q, mm[u]);
+        store4<STREAM>(nu, q, vv[u]);
       }
     }
   } else {
@@ -1437,10 +1462,13 @@ extern "C" int gs_preprocess_bwd_adam(void* stream, int64_t n, int sh_k, int sh_
   A.eps = (float)eps;
   (void)cx;
   (void)cy;
-#define GS_PRE_BWD_ADAM(D)                                                                                       \
-  hipLaunchKernelGGL(preprocess_bwd_adam_kernel<D>, dim3(div_up(n, 64)), dim3(64), 0, (hipStream_t)stream, n,     \
+#define GS_PRE_BWD_ADAM1(D, STREAM)                                                                              \
+  hipLaunchKernelGGL((preprocess_bwd_adam_kernel<D, STREAM>), dim3(div_up(n, 64)), dim3(64), 0, (hipStream_t)stream, n, \
                      sh_k, means, scales, quats, opacities, sh_coeffs, w2c, fx, fy, grad_records, M, A, active, valid, \
                      radii, focal, pixel_scale, grad_accum, denom, max_radii)
+  const bool stream_sh = 3 * n * 3 * sh_k * (int64_t)sizeof(float) >= kStreamBytes;
+#define GS_PRE_BWD_ADAM(D) \
+  if (stream_sh) GS_PRE_BWD_ADAM1(D, true); else GS_PRE_BWD_ADAM1(D, false)
   switch (sh_degree) {
     case 0: GS_PRE_BWD_ADAM(0); break;
     case 1: GS_PRE_BWD_ADAM(1); break;
@@ -1448,6 +1476,7 @@ extern "C" int gs_preprocess_bwd_adam(void* stream, int64_t n, int sh_k, int sh_
     default: GS_PRE_BWD_ADAM(3); break;
   }
 #undef GS_PRE_BWD_ADAM
+#undef GS_PRE_BWD_ADAM1
   GS_LAUNCH_CHECK("preprocess_bwd_adam_kernel");
   return GS_OK;
 }
