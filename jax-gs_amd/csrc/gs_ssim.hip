@@ -9,15 +9,22 @@
 //   map = (2 mu1 mu2 + C1)(2 s12 + C2) / ((mu1^2 + mu2^2 + C1)(s11 + s22 + C2)),
 //   C1 = 0.01^2, C2 = 0.03^2, clipped to [-1, 1]; ssim = mean over H x W x C.
 //
-// Forward (one launch + a final sum): a workgroup owns 16 x 54 outputs of every channel.
-// The vertical pass runs over 64 columns (54 + 2 x 5 halo): each thread takes one
-// column and 4 output rows, reads the 14 input rows it needs once and keeps the five
-// blurred products (x, y, x^2, y^2, x y) in registers; they meet in LDS, where the
-// horizontal pass (each thread 4 adjacent outputs of one row, 128-bit LDS reads of
-// its 14-column window) completes the blur.  Per output the map, |x - y| and, when a
-// gradient is wanted, the map's derivatives with respect to (mu1, blur(x^2),
-// blur(x y)) -- divided by the count and gated by the clip -- are formed; the
-// derivatives go to three planes of the workspace.
+// Forward (one launch + a final sum): a workgroup owns 8 x 116 outputs of every channel.
+// The vertical pass runs over 128 columns (116 + the halo): each thread takes one column and
+// 4 output rows, reads the 14 input rows it needs once (rows are the wave's, so their
+// addresses are scalar) and keeps the five blurred products (x, y, x^2, y^2, x y) in
+// registers; they meet in LDS, where the horizontal pass (each thread 4 adjacent outputs of
+// one row, 128-bit LDS reads of its 14-column window) completes the blur.  Per output the
+// map and, when a gradient is wanted, its derivatives with respect to (mu1, blur(x^2),
+// blur(x y)) -- divided by the count and gated by the clip -- are formed; a group of four
+// goes to the three planes of the workspace as 16-byte stores.  |x - y| comes from the rows
+// that the vertical pass holds.
+// What bounds it: the two passes are 2 x 55 of some 170 vector instructions per value, about
+// 27 us at 1920x1080 x 3, and reading the images with writing the planes (125 MB) 25 us.  A
+// tile of 16 x 54 (halo and idle lanes: 30 % more of both passes, now 10 %) with the planes and
+// the gradient staged in LDS took 72 us forward and 52 backward; this takes 47.5 and 32.5.
+// Prefetching the next channel's rows beside the horizontal pass costs the forward more
+// registers than it hides (53 us, with 3 waves per SIMD 51); the backward's three maps do it.
 // Backward: dL/dx = blur(d/dmu1) + 2 x blur(d/dblur(x^2)) + y blur(d/dblur(x y)) (the
 // blur is a correlation with a symmetric kernel and zero padding, so it is its own
 // adjoint), scaled by the cotangent of the mean SSIM, plus the L1 cotangent times
@@ -30,10 +37,10 @@ namespace {
 
 constexpr int kSR = 5;                   // window radius
 constexpr int kSTaps = 2 * kSR + 1;      // 11 taps
-constexpr int kSTH = 16;                 // output rows per workgroup
-constexpr int kSCols = 64;               // columns of the vertical pass
-constexpr int kSTW = kSCols - 2 * kSR;   // 54 output columns per workgroup
-constexpr int kSPad = kSCols + 4;        // LDS row (the last window reads 2 columns past 64)
+constexpr int kSTH = 8;                  // output rows per workgroup
+constexpr int kSCols = 128;              // columns of the vertical pass
+constexpr int kSTW = 116;                // output columns per workgroup: 29 groups of 4, all 14-column windows inside kSCols
+constexpr int kSRows = 4 + 2 * kSR;      // input rows of a thread's four output rows
 constexpr float kC1 = 0.01f * 0.01f;
 constexpr float kC2 = 0.03f * 0.03f;
 
@@ -43,33 +50,30 @@ struct Taps {
 
 __device__ inline float tie_step(float z) { return z > 0.0f ? 1.0f : (z == 0.0f ? 0.5f : 0.0f); }
 
-// Vertical pass of NM maps for image column col: acc[m][o] = sum_k w_k v_m(row0 + o + k),
-// o < 4, where v_m(r) = load(m, r) inside the image and 0 outside.
-template <int NM, typename Load>
-__device__ inline void vertical4(const Taps& t, int row0, int H, bool col_in, Load load, float (&acc)[NM][4]) {
+// What a thread of the vertical pass reads of one map: rows row0 .. row0 + 13 of its column.  The
+// rows are the wave's (scalar addresses); rows and columns outside the image are read at their
+// nearest inside one (the caller zeroes them, in the workgroups that have any).
+struct Column {
+  int off;     // element of (row 0, the thread's column, channel 0), column clamped
+  int row0;    // wave-uniform
+  int H;
+  int stride;  // elements from row to row
+};
+__device__ inline void load_rows(const float* __restrict__ p, const Column& c, float (&v)[kSRows]) {
 #pragma unroll
-  for (int m = 0; m < NM; ++m)
-#pragma unroll
-    for (int o = 0; o < 4; ++o) acc[m][o] = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 4 + 2 * kSR; ++i) {
-    const int r = row0 + i;
-    float v[NM];
-    load(col_in && r >= 0 && r < H, r, v);
-#pragma unroll
-    for (int o = 0; o < 4; ++o) {
-      const int k = i - o;
-      if (k >= 0 && k < kSTaps) {
-#pragma unroll
-        for (int m = 0; m < NM; ++m) acc[m][o] = fmaf(t.w[k], v[m], acc[m][o]);
-      }
-    }
+  for (int i = 0; i < kSRows; ++i) {
+    const int r = min(max(c.row0 + i, 0), c.H - 1);
+    v[i] = (p + (int64_t)r * c.stride)[c.off];
   }
+}
+__device__ inline void zero_outside(const Column& c, bool col_in, float (&v)[kSRows]) {
+#pragma unroll
+  for (int i = 0; i < kSRows; ++i) v[i] = col_in && c.row0 + i >= 0 && c.row0 + i < c.H ? v[i] : 0.0f;
 }
 
 // Horizontal pass from LDS row `row` of NM maps: out[m][o] = sum_k w_k V[m][row][c0 + o + k].
 template <int NM>
-__device__ inline void horizontal4(const Taps& t, const float (*V)[kSTH][kSPad], int row, int c0, float (&out)[NM][4]) {
+__device__ inline void horizontal4(const Taps& t, const float (*V)[kSTH][kSCols], int row, int c0, float (&out)[NM][4]) {
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
     float win[16];
@@ -106,44 +110,63 @@ __device__ inline float block_sum256(float v, float* red) {
 // the halo rows two vertically adjacent tiles share are fetched once.
 __device__ inline int ssim_tile_of_block(int b, int T) { return (b & 7) * ((T + 7) >> 3) + (b >> 3); }
 
-// Forward, CC channels (1..4), one channel at a time (the next channel's loads hit the
-// cache).  The gradient maps of a channel are staged in LDS and leave as whole rows.
+// Forward, CC channels (1..4), one channel at a time: the next channel's rows are loaded
+// into registers while the horizontal pass of the current one runs.
 template <int CC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l1_ssim_fwd_kernel(
     int H, int W, int TX, int T, const float* __restrict__ x, const float* __restrict__ y, Taps taps,
-    float inv_count, float* __restrict__ gmap, float2* __restrict__ partial) {
-  __shared__ __align__(16) float V[5][kSTH][kSPad];
-  __shared__ float Gs[3][kSTH][kSTW];
+    float inv_count, float* __restrict__ gmap, bool vec, float2* __restrict__ partial) {
+  __shared__ __align__(16) float V[5][kSTH][kSCols];
   __shared__ float red[4];
   const int tile = ssim_tile_of_block(blockIdx.x, T);
   if (tile >= T) return;
   const int tid = threadIdx.x;
   const int ox = (tile % TX) * kSTW;  // first output column
   const int r0 = (tile / TX) * kSTH;  // first output row
-  // columns 64..67 of every LDS row feed only outputs past the tile: keep them finite
-  for (int i = tid; i < 5 * kSTH * 4; i += 256) V[i / (kSTH * 4)][(i / 4) % kSTH][kSCols + (i & 3)] = 0.0f;
-  const int vj = tid & 63, vq = tid >> 6;  // vertical pass: column, group of 4 rows
+  // vertical pass: column, and the wave's group of 4 rows
+  const int vj = tid & 127, vq = __builtin_amdgcn_readfirstlane(tid >> 7);
   const int vcol = ox - kSR + vj;
   const bool vcol_in = vcol >= 0 && vcol < W;
-  const int hr = tid >> 4, hs = tid & 15;  // horizontal pass: row, group of 4 columns
-  const bool h_on = 4 * hs < kSTW;
+  const Column col{min(max(vcol, 0), W - 1) * CC, r0 + 4 * vq - kSR, H, W * CC};
+  const bool border = ox < kSR || ox - kSR + kSCols > W || r0 < kSR || r0 + kSTH + kSR > H;
+  const bool vout = vj >= kSR && vj < kSR + kSTW && vcol < W;  // an output column of this tile
+  const int hr = tid >> 5, hs = tid & 31;  // horizontal pass: row, group of 4 columns
+  const int orow = r0 + hr, ocol = ox + 4 * hs;
+  const bool h_on = 4 * hs < kSTW && orow < H && ocol < W;
   const int plane = H * W * CC;  // one gradient map, channel-planar [CC][H][W]
   float l1_acc = 0.0f, ss_acc = 0.0f;
+  float xv[kSRows], yv[kSRows];
 #pragma unroll 1
   for (int ch = 0; ch < CC; ++ch) {
+    load_rows(x + ch, col, xv);
+    load_rows(y + ch, col, yv);
+    if (border) {
+      zero_outside(col, vcol_in, xv);
+      zero_outside(col, vcol_in, yv);
+    }
     float a[5][4];
-    vertical4<5>(taps, r0 + 4 * vq - kSR, H, vcol_in,
-                 [&](bool in, int r, float* v) {
-                   const int o = (r * W + vcol) * CC + ch;  // 3 * count < 2^31 (checked by the host)
-                   const float xv = in ? x[o] : 0.0f, yv = in ? y[o] : 0.0f;
-                   v[0] = xv;
-                   v[1] = yv;
-                   v[2] = xv * xv;
-                   v[3] = yv * yv;
-                   v[4] = xv * yv;
-                 },
-                 a);
-    if (ch > 0) __syncthreads();  // the previous channel is done with V and Gs
+#pragma unroll
+    for (int m = 0; m < 5; ++m)
+#pragma unroll
+      for (int o = 0; o < 4; ++o) a[m][o] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kSRows; ++i) {
+      const float v[5] = {xv[i], yv[i], xv[i] * xv[i], yv[i] * yv[i], xv[i] * yv[i]};
+#pragma unroll
+      for (int o = 0; o < 4; ++o) {
+        const int k = i - o;
+        if (k >= 0 && k < kSTaps) {
+#pragma unroll
+          for (int m = 0; m < 5; ++m) a[m][o] = fmaf(taps.w[k], v[m], a[m][o]);
+        }
+      }
+    }
+    // rows outside the image hold zeros in both
+    if (vout) {
+#pragma unroll
+      for (int o = 0; o < 4; ++o) l1_acc += fabsf(xv[kSR + o] - yv[kSR + o]);
+    }
+    if (ch > 0) __syncthreads();  // the previous channel is done with V
 #pragma unroll
     for (int m = 0; m < 5; ++m)
 #pragma unroll
@@ -152,11 +175,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
     if (h_on) {
       float b[5][4];
       horizontal4<5>(taps, V, hr, 4 * hs, b);
-      const int orow = r0 + hr;
+      float G0[4], G1[4], G2[4];
 #pragma unroll
       for (int o = 0; o < 4; ++o) {
-        const int tc = 4 * hs + o, ocol = ox + tc;
-        if (tc >= kSTW || ocol >= W || orow >= H) continue;
         const float mu1 = b[0][o], mu2 = b[1][o];
         const float m11 = mu1 * mu1, m22 = mu2 * mu2, m12 = mu1 * mu2;
         const float d11 = b[2][o] - m11;
@@ -168,9 +189,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
         // one reciprocal for the three quotients (den >= C1 C2 > 0; ~1 ulp)
         const float rden = __builtin_amdgcn_rcpf(den);
         const float raw = num * rden;
-        ss_acc += fminf(1.0f, fmaxf(-1.0f, raw));
-        const int p = (orow * W + ocol) * CC + ch;
-        l1_acc += fabsf(x[p] - y[p]);
+        if (ocol + o < W) ss_acc += fminf(1.0f, fmaxf(-1.0f, raw));
         // d map / d(mu1, blur(x^2), blur(x y)), times the clip gate and 1 / count
         const float G = inv_count * (tie_step(raw + 1.0f) * tie_step(1.0f - raw));
         const float dnum = G * rden, dden = -(G * raw) * rden;
@@ -179,19 +198,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
         const float dm12 = 2.0f * dA - de12;
         const float de11 = dD * tie_step(d11);
         const float dm11 = dCc - de11;
-        Gs[0][hr][tc] = 2.0f * mu1 * dm11 + mu2 * dm12;
-        Gs[1][hr][tc] = de11;
-        Gs[2][hr][tc] = de12;
+        G0[o] = 2.0f * mu1 * dm11 + mu2 * dm12;
+        G1[o] = de11;
+        G2[o] = de12;
       }
-    }
-    if (gmap != nullptr) {
-      __syncthreads();
-      // wave w writes rows w, w + 4, ... of the 3 x 16 staged rows, one value per lane
-      const int lane = tid & 63, wv = tid >> 6;
-      const int ncol = min(kSTW, W - ox);
-      for (int row = wv; row < 3 * kSTH; row += 4) {
-        const int m = row / kSTH, rr = row % kSTH, orow = r0 + rr;
-        if (orow < H && lane < ncol) gmap[m * plane + (ch * H + orow) * W + ox + lane] = Gs[m][rr][lane];
+      if (gmap != nullptr) {
+        float* __restrict__ g = gmap + (ch * H + orow) * W + ocol;
+        if (vec) {  // W a multiple of 4: whole groups, aligned
+          *reinterpret_cast<float4*>(g) = make_float4(G0[0], G0[1], G0[2], G0[3]);
+          *reinterpret_cast<float4*>(g + plane) = make_float4(G1[0], G1[1], G1[2], G1[3]);
+          *reinterpret_cast<float4*>(g + 2 * (int64_t)plane) = make_float4(G2[0], G2[1], G2[2], G2[3]);
+        } else {
+#pragma unroll
+          for (int o = 0; o < 4; ++o) {
+            if (ocol + o >= W) break;
+            g[o] = G0[o];
+            g[plane + o] = G1[o];
+            g[2 * (int64_t)plane + o] = G2[o];
+          }
+        }
       }
     }
   }
@@ -227,69 +252,98 @@ __global__ __launch_bounds__(1024) void l1_ssim_sum_kernel(const float2* __restr
   }
 }
 
-// Backward: the image gradient of the tile (every channel) is staged in LDS and leaves
-// as whole rows.
+// Backward: a thread of the horizontal pass holds its four pixels' values of every channel
+// (4 CC contiguous floats) and stores their gradients; the next channel's rows of the maps are
+// loaded while the horizontal pass of the current one runs.
 template <int CC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l1_ssim_bwd_kernel(
     int H, int W, int TX, int T, const float* __restrict__ x, const float* __restrict__ y, Taps taps,
-    float inv_count, const float* __restrict__ gmap, const float* __restrict__ grad_out,
+    float inv_count, const float* __restrict__ gmap, const float* __restrict__ grad_out, bool vec,
     float* __restrict__ grad) {
-  __shared__ __align__(16) float V[3][kSTH][kSPad];
-  __shared__ float Go[kSTH][kSTW * CC];
+  __shared__ __align__(16) float V[3][kSTH][kSCols];
   const int tile = ssim_tile_of_block(blockIdx.x, T);
   if (tile >= T) return;
   const int tid = threadIdx.x;
   const int ox = (tile % TX) * kSTW, r0 = (tile / TX) * kSTH;
-  for (int i = tid; i < 3 * kSTH * 4; i += 256) V[i / (kSTH * 4)][(i / 4) % kSTH][kSCols + (i & 3)] = 0.0f;
-  const int vj = tid & 63, vq = tid >> 6;
+  const int vj = tid & 127, vq = __builtin_amdgcn_readfirstlane(tid >> 7);
   const int vcol = ox - kSR + vj;
   const bool vcol_in = vcol >= 0 && vcol < W;
-  const int hr = tid >> 4, hs = tid & 15;
-  const bool h_on = 4 * hs < kSTW;
-  const int plane = H * W * CC;
+  const Column col{min(max(vcol, 0), W - 1), r0 + 4 * vq - kSR, H, W};
+  const bool border = ox < kSR || ox - kSR + kSCols > W || r0 < kSR || r0 + kSTH + kSR > H;
+  const int hr = tid >> 5, hs = tid & 31;
+  const int orow = r0 + hr, ocol = ox + 4 * hs;
+  const bool h_on = 4 * hs < kSTW && orow < H && ocol < W;
+  const int64_t plane = (int64_t)H * W * CC;
   const float g_l1 = grad_out[0] * inv_count, g_ss = grad_out[1];
-#pragma unroll 1
+  const int64_t p = ((int64_t)orow * W + ocol) * CC;  // the thread's first value
+  const int nval = h_on ? min(4, W - ocol) * CC : 0;
+  float v[3][kSRows];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) load_rows(gmap + m * plane, col, v[m]);
+  float xq[4 * CC], yq[4 * CC];
+  if (vec) {
+    if (nval > 0) {
+#pragma unroll
+      for (int q = 0; q < CC; ++q) {
+        const float4 fx = reinterpret_cast<const float4*>(x + p)[q], fy = reinterpret_cast<const float4*>(y + p)[q];
+        xq[4 * q] = fx.x, xq[4 * q + 1] = fx.y, xq[4 * q + 2] = fx.z, xq[4 * q + 3] = fx.w;
+        yq[4 * q] = fy.x, yq[4 * q + 1] = fy.y, yq[4 * q + 2] = fy.z, yq[4 * q + 3] = fy.w;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4 * CC; ++q) {
+      xq[q] = q < nval ? x[p + q] : 0.0f;
+      yq[q] = q < nval ? y[p + q] : 0.0f;
+    }
+  }
+#pragma unroll
   for (int ch = 0; ch < CC; ++ch) {
+    if (border) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) zero_outside(col, vcol_in, v[m]);
+    }
     float a[3][4];
-    vertical4<3>(taps, r0 + 4 * vq - kSR, H, vcol_in,
-                 [&](bool in, int r, float* v) {
-                   const int q = (ch * H + r) * W + vcol;
-                   v[0] = in ? gmap[q] : 0.0f;
-                   v[1] = in ? gmap[plane + q] : 0.0f;
-                   v[2] = in ? gmap[2 * plane + q] : 0.0f;
-                 },
-                 a);
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int o = 0; o < 4; ++o) {
+        a[m][o] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kSTaps; ++k) a[m][o] = fmaf(taps.w[k], v[m][o + k], a[m][o]);
+      }
     if (ch > 0) __syncthreads();
 #pragma unroll
     for (int m = 0; m < 3; ++m)
 #pragma unroll
       for (int o = 0; o < 4; ++o) V[m][4 * vq + o][vj] = a[m][o];
     __syncthreads();
+    if (ch + 1 < CC) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) load_rows(gmap + m * plane + (int64_t)(ch + 1) * H * W, col, v[m]);
+    }
     if (h_on) {
       float b[3][4];
       horizontal4<3>(taps, V, hr, 4 * hs, b);
-      const int orow = r0 + hr;
 #pragma unroll
       for (int o = 0; o < 4; ++o) {
-        const int tc = 4 * hs + o, ocol = ox + tc;
-        if (tc >= kSTW || ocol >= W || orow >= H) continue;
-        const int p = (orow * W + ocol) * CC + ch;
-        const float xv = x[p], yv = y[p], d = xv - yv;
+        const float xv = xq[o * CC + ch], yv = yq[o * CC + ch], d = xv - yv;
         const float sg = d > 0.0f ? 1.0f : (d < 0.0f ? -1.0f : 0.0f);
         const float gs = b[0][o] + 2.0f * xv * b[1][o] + yv * b[2][o];
-        Go[hr][tc * CC + ch] = g_ss * gs + g_l1 * sg;
+        xq[o * CC + ch] = g_ss * gs + g_l1 * sg;  // the value is done with
       }
     }
   }
-  __syncthreads();
-  // wave w writes rows w, w + 4, ...: a row is min(54, W - ox) * CC contiguous values
-  const int lane = tid & 63, wv = tid >> 6;
-  const int wcols = min(kSTW, W - ox) * CC;
-  for (int rr = wv; rr < kSTH; rr += 4) {
-    const int orow = r0 + rr;
-    if (orow >= H) break;
-    float* __restrict__ dst = grad + (orow * W + ox) * CC;
-    for (int cc = lane; cc < wcols; cc += 64) dst[cc] = Go[rr][cc];
+  if (vec) {
+    if (nval > 0) {
+#pragma unroll
+      for (int q = 0; q < CC; ++q)
+        reinterpret_cast<float4*>(grad + p)[q] = make_float4(xq[4 * q], xq[4 * q + 1], xq[4 * q + 2], xq[4 * q + 3]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4 * CC; ++q)
+      if (q < nval) grad[p + q] = xq[q];
   }
 }
 
@@ -490,6 +544,11 @@ struct SsimLayout {
   size_t gmap_off, part_off, total;
 };
 
+// Groups of four columns are whole and 16-byte aligned in arrays of this width.
+bool whole_groups(int width, const void* a, const void* b, const void* c) {
+  return width % 4 == 0 && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0;
+}
+
 SsimLayout ssim_layout(int H, int W, int C) {
   SsimLayout L;
   L.count = (int64_t)H * W * C;
@@ -526,12 +585,13 @@ extern "C" int gs_l1_ssim(void* stream, int height, int width, int channels, con
   const float inv = (float)(1.0 / (double)L.count);
   float2* part = (float2*)(ws + L.part_off);
   float* gmap = with_grad ? (float*)(ws + L.gmap_off) : nullptr;
+  const bool vec = whole_groups(width, gmap, nullptr, nullptr);
   const Taps taps = make_taps();
   switch (channels) {
-    case 1: hipLaunchKernelGGL(l1_ssim_fwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
-    case 2: hipLaunchKernelGGL(l1_ssim_fwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
-    case 3: hipLaunchKernelGGL(l1_ssim_fwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
-    default: hipLaunchKernelGGL(l1_ssim_fwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
+    case 1: hipLaunchKernelGGL(l1_ssim_fwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
+    case 2: hipLaunchKernelGGL(l1_ssim_fwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
+    case 3: hipLaunchKernelGGL(l1_ssim_fwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
+    default: hipLaunchKernelGGL(l1_ssim_fwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
   }
   GS_LAUNCH_CHECK("l1_ssim_fwd_kernel");
   hipLaunchKernelGGL(l1_ssim_sum_kernel, dim3(1), dim3(1024), 0, s, (const float2*)part, L.T, inv, out);
@@ -553,12 +613,13 @@ extern "C" int gs_l1_ssim_bwd(void* stream, int height, int width, int channels,
   hipStream_t s = (hipStream_t)stream;
   const float inv = (float)(1.0 / (double)L.count);
   const float* gmap = (const float*)((const char*)workspace + L.gmap_off);
+  const bool vec = whole_groups(width, pred, target, grad_pred);
   const Taps taps = make_taps();
   switch (channels) {
-    case 1: hipLaunchKernelGGL(l1_ssim_bwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, grad_pred); break;
-    case 2: hipLaunchKernelGGL(l1_ssim_bwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, grad_pred); break;
-    case 3: hipLaunchKernelGGL(l1_ssim_bwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, grad_pred); break;
-    default: hipLaunchKernelGGL(l1_ssim_bwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, grad_pred); break;
+    case 1: hipLaunchKernelGGL(l1_ssim_bwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
+    case 2: hipLaunchKernelGGL(l1_ssim_bwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
+    case 3: hipLaunchKernelGGL(l1_ssim_bwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
+    default: hipLaunchKernelGGL(l1_ssim_bwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
   }
   GS_LAUNCH_CHECK("l1_ssim_bwd_kernel");
   return GS_OK;
