@@ -90,7 +90,8 @@ const char* gs_last_error(void);
  * builds it; gs_window_from_bins stays for lists binned without it).  14: gs_composite_bwd
  * and gs_composite_bwd_l1 take a gs_clear_list_t; gs_preprocess_bwd and
  * gs_preprocess_bwd_w2c take zeroed.  Added since, with every call of 14 as it was:
- * gs_composite_segments_size, gs_composite_fwd_seg, gs_composite_bwd_seg. */
+ * gs_composite_segments_size, gs_composite_fwd_seg, gs_composite_bwd_seg; gs_l1_ssim_loss,
+ * gs_l1_ssim_loss_bwd. */
 int gs_abi_version(void);
 
 /* Projection + covariance + SH colour for every Gaussian.
@@ -485,6 +486,20 @@ int gs_l1_ssim_window_bwd(void* stream, int height, int width, int channels, int
  * grad_out of gs_l1_ssim_bwd; max passes half at a tie), terms[4] = 1 - 2 d_ssim (the
  * reported SSIM, trainer.py:30).  Device arrays, one launch. */
 int gs_l1_ssim_terms(void* stream, const float* l1_ssim, double lambda_ssim, float* terms);
+
+/* gs_l1_ssim and the trainer's loss from its means in the same launches: l1_ssim[2] as gs_l1_ssim's
+ * out, terms[5] as gs_l1_ssim_terms, and the total, the L1 mean and d_ssim as scalars of their own
+ * (each of these four may be NULL).  Any lambda. */
+int gs_l1_ssim_loss(void* stream, int height, int width, int channels, const float* pred, const float* target,
+                    double lambda_ssim, float* l1_ssim, float* terms, float* total, float* l1, float* d_ssim,
+                    int with_grad, void* workspace, size_t workspace_bytes);
+
+/* gs_l1_ssim_bwd with the cotangents of (l1, ssim) formed on the device from those of
+ * gs_l1_ssim_loss's total, l1 and d_ssim (device scalars, NULL for none; max passes half at its tie)
+ * and its l1_ssim. */
+int gs_l1_ssim_loss_bwd(void* stream, int height, int width, int channels, const float* pred, const float* target,
+                        double lambda_ssim, const float* l1_ssim, const float* g_total, const float* g_l1,
+                        const float* g_d_ssim, const void* workspace, size_t workspace_bytes, float* grad_pred);
 
 /* One Adam step, in place, of num_arrays (<= 8) float32 parameter arrays, each with
  * its gradient and first/second moments (same sizes), counts[i] elements laid out as

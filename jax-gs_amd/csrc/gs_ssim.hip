@@ -225,9 +225,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
   if (tid == 0) partial[tile] = make_float2(l1s, sss);
 }
 
-// out[0] = sum of |x - y| / count, out[1] = sum of the clipped map / count.
+// trainer.py:18-26 from the two means; same float32 operations as the host-side formula.
+struct LossOut {
+  float lam, one_minus_lam;
+  float *terms, *total, *l1, *d;  // each may be NULL
+};
+__device__ inline void loss_terms(float l1, float ssim, const LossOut& o) {
+  const float half = (1.0f - ssim) / 2.0f;
+  const float d = fmaxf(0.0f, half), total = o.one_minus_lam * l1 + o.lam * d;
+  if (o.terms != nullptr) {
+    o.terms[0] = d;
+    o.terms[1] = total;
+    o.terms[2] = o.one_minus_lam;
+    const float gate = half > 0.0f ? 1.0f : (half == 0.0f ? 0.5f : 0.0f);
+    o.terms[3] = -(o.lam * 0.5f) * gate;
+    o.terms[4] = 1.0f - d * 2.0f;
+  }
+  if (o.total != nullptr) *o.total = total;
+  if (o.l1 != nullptr) *o.l1 = l1;
+  if (o.d != nullptr) *o.d = d;
+}
+
+// out[0] = sum of |x - y| / count, out[1] = sum of the clipped map / count; LOSS: and the
+// trainer's loss from them.
+template <bool LOSS>
 __global__ __launch_bounds__(1024) void l1_ssim_sum_kernel(const float2* __restrict__ partial, int nb,
-                                                           float inv_count, float* __restrict__ out) {
+                                                           float inv_count, float* __restrict__ out,
+                                                           const LossOut loss) {
   __shared__ float red[2][16];
   float a = 0.0f, b = 0.0f;
   for (int i = threadIdx.x; i < nb; i += 1024) {
@@ -249,7 +273,35 @@ __global__ __launch_bounds__(1024) void l1_ssim_sum_kernel(const float2* __restr
     float s = 0.0f;
     for (int w = 0; w < 16; ++w) s += red[threadIdx.x][w];
     out[threadIdx.x] = s * inv_count;
+    const float ssim = __shfl(s * inv_count, 1, 64);
+    if (LOSS && threadIdx.x == 0) loss_terms(s * inv_count, ssim, loss);
   }
+}
+
+// The cotangents of (l1, ssim) that the backward starts from: an array of two, or formed from
+// those of the trainer's loss, of its l1 and of its d_ssim (each a device scalar, NULL for none)
+// as autodiff of trainer.py:18-26 forms them (max passes half at a tie).
+struct LossCot {
+  const float* grad_out;
+  const float* l1_ssim;
+  const float *total, *l1, *d;
+  float lam, one_minus_lam;
+};
+__device__ inline void loss_cot(const LossCot& c, float& g_l1, float& g_ss) {
+  if (c.grad_out != nullptr) {
+    g_l1 = c.grad_out[0];
+    g_ss = c.grad_out[1];
+    return;
+  }
+  const float half = (1.0f - c.l1_ssim[1]) / 2.0f;
+  const float gate = half > 0.0f ? 1.0f : (half == 0.0f ? 0.5f : 0.0f);
+  g_l1 = c.l1 != nullptr ? *c.l1 : 0.0f;
+  float gd = c.d != nullptr ? *c.d : 0.0f;
+  if (c.total != nullptr) {
+    g_l1 += *c.total * c.one_minus_lam;
+    gd += *c.total * c.lam;
+  }
+  g_ss = -(gd * gate / 2.0f);
 }
 
 // Backward: a thread of the horizontal pass holds its four pixels' values of every channel
@@ -258,7 +310,7 @@ __global__ __launch_bounds__(1024) void l1_ssim_sum_kernel(const float2* __restr
 template <int CC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l1_ssim_bwd_kernel(
     int H, int W, int TX, int T, const float* __restrict__ x, const float* __restrict__ y, Taps taps,
-    float inv_count, const float* __restrict__ gmap, const float* __restrict__ grad_out, bool vec,
+    float inv_count, const float* __restrict__ gmap, const LossCot cot, bool vec,
     float* __restrict__ grad) {
   __shared__ __align__(16) float V[3][kSTH][kSCols];
   const int tile = ssim_tile_of_block(blockIdx.x, T);
@@ -274,7 +326,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
   const int orow = r0 + hr, ocol = ox + 4 * hs;
   const bool h_on = 4 * hs < kSTW && orow < H && ocol < W;
   const int64_t plane = (int64_t)H * W * CC;
-  const float g_l1 = grad_out[0] * inv_count, g_ss = grad_out[1];
+  float g_l1, g_ss;
+  loss_cot(cot, g_l1, g_ss);
+  g_l1 *= inv_count;
   const int64_t p = ((int64_t)orow * W + ocol) * CC;  // the thread's first value
   const int nval = h_on ? min(4, W - ocol) * CC : 0;
   float v[3][kSRows];
@@ -347,22 +401,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
   }
 }
 
-// trainer.py:18-26 from the two means: terms[0] = d_ssim = max(0, (1 - ssim) / 2),
-// terms[1] = total = (1 - lambda) l1 + lambda d_ssim, and the cotangents of (l1, ssim)
-// for a unit cotangent of the total: terms[2] = 1 - lambda, terms[3] = -lambda/2 times
-// max's derivative (1 above 0, 1/2 at 0, as lax.max), and terms[4] = the reported metric
-// 1 - 2 d_ssim (trainer.py:30).  Same float32 operations as the host-side formula.
-__global__ void l1_ssim_terms_kernel(const float* __restrict__ l1_ssim, float lam, float one_minus_lam,
-                                     float* __restrict__ terms) {
-  const float l1 = l1_ssim[0], ssim = l1_ssim[1];
-  const float half = (1.0f - ssim) / 2.0f;
-  const float d = fmaxf(0.0f, half);
-  terms[0] = d;
-  terms[1] = one_minus_lam * l1 + lam * d;
-  terms[2] = one_minus_lam;
-  const float gate = half > 0.0f ? 1.0f : (half == 0.0f ? 0.5f : 0.0f);
-  terms[3] = -(lam * 0.5f) * gate;
-  terms[4] = 1.0f - d * 2.0f;
+__global__ void l1_ssim_terms_kernel(const float* __restrict__ l1_ssim, const LossOut loss) {
+  loss_terms(l1_ssim[0], l1_ssim[1], loss);
 }
 
 // ---------------------------------------------------------------------------------
@@ -571,15 +611,17 @@ extern "C" size_t gs_l1_ssim_workspace_size(int height, int width, int channels)
   return ssim_layout(height, width, channels).total;
 }
 
-extern "C" int gs_l1_ssim(void* stream, int height, int width, int channels, const float* pred,
-                          const float* target, float* out, int with_grad, void* workspace, size_t workspace_bytes) {
-  GS_REQUIRE(height > 0 && width > 0 && channels > 0 && channels <= 4, "gs_l1_ssim: bad image shape %dx%dx%d",
+namespace {
+int l1_ssim_fwd_run(const char* name, void* stream, int height, int width, int channels, const float* pred,
+                    const float* target, float* out, int with_grad, void* workspace, size_t workspace_bytes,
+                    const LossOut* loss) {
+  GS_REQUIRE(height > 0 && width > 0 && channels > 0 && channels <= 4, "%s: bad image shape %dx%dx%d", name,
              height, width, channels);
-  GS_REQUIRE(pred && target && out && workspace, "gs_l1_ssim: NULL argument");
+  GS_REQUIRE(pred && target && out && workspace, "%s: NULL argument", name);
   GS_REQUIRE(3 * (int64_t)height * width * channels < ((int64_t)1 << 31),
-             "gs_l1_ssim: image %dx%dx%d too large", height, width, channels);
+             "%s: image %dx%dx%d too large", name, height, width, channels);
   const SsimLayout L = ssim_layout(height, width, channels);
-  GS_REQUIRE(workspace_bytes >= L.total, "gs_l1_ssim: workspace of %zu bytes, %zu needed", workspace_bytes, L.total);
+  GS_REQUIRE(workspace_bytes >= L.total, "%s: workspace of %zu bytes, %zu needed", name, workspace_bytes, L.total);
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
   const float inv = (float)(1.0 / (double)L.count);
@@ -594,21 +636,41 @@ extern "C" int gs_l1_ssim(void* stream, int height, int width, int channels, con
     default: hipLaunchKernelGGL(l1_ssim_fwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
   }
   GS_LAUNCH_CHECK("l1_ssim_fwd_kernel");
-  hipLaunchKernelGGL(l1_ssim_sum_kernel, dim3(1), dim3(1024), 0, s, (const float2*)part, L.T, inv, out);
+  if (loss != nullptr)
+    hipLaunchKernelGGL(l1_ssim_sum_kernel<true>, dim3(1), dim3(1024), 0, s, (const float2*)part, L.T, inv, out, *loss);
+  else
+    hipLaunchKernelGGL(l1_ssim_sum_kernel<false>, dim3(1), dim3(1024), 0, s, (const float2*)part, L.T, inv, out,
+                       LossOut{});
   GS_LAUNCH_CHECK("l1_ssim_sum_kernel");
   return GS_OK;
 }
+}  // namespace
 
-extern "C" int gs_l1_ssim_bwd(void* stream, int height, int width, int channels, const float* pred,
-                              const float* target, const float* grad_out, const void* workspace,
-                              size_t workspace_bytes, float* grad_pred) {
+extern "C" int gs_l1_ssim(void* stream, int height, int width, int channels, const float* pred,
+                          const float* target, float* out, int with_grad, void* workspace, size_t workspace_bytes) {
+  return l1_ssim_fwd_run("gs_l1_ssim", stream, height, width, channels, pred, target, out, with_grad, workspace,
+                         workspace_bytes, nullptr);
+}
+
+extern "C" int gs_l1_ssim_loss(void* stream, int height, int width, int channels, const float* pred,
+                               const float* target, double lambda_ssim, float* l1_ssim, float* terms, float* total,
+                               float* l1, float* d_ssim, int with_grad, void* workspace, size_t workspace_bytes) {
+  const LossOut loss{(float)lambda_ssim, (float)(1.0 - lambda_ssim), terms, total, l1, d_ssim};
+  return l1_ssim_fwd_run("gs_l1_ssim_loss", stream, height, width, channels, pred, target, l1_ssim, with_grad,
+                         workspace, workspace_bytes, &loss);
+}
+
+namespace {
+int l1_ssim_bwd_run(const char* name, void* stream, int height, int width, int channels, const float* pred,
+                    const float* target, const LossCot& cot, const void* workspace, size_t workspace_bytes,
+                    float* grad_pred) {
   GS_REQUIRE(height > 0 && width > 0 && channels > 0 && channels <= 4,
-             "gs_l1_ssim_bwd: bad image shape %dx%dx%d", height, width, channels);
-  GS_REQUIRE(pred && target && grad_out && workspace && grad_pred, "gs_l1_ssim_bwd: NULL argument");
+             "%s: bad image shape %dx%dx%d", name, height, width, channels);
+  GS_REQUIRE(pred && target && (cot.grad_out || cot.l1_ssim) && workspace && grad_pred, "%s: NULL argument", name);
   GS_REQUIRE(3 * (int64_t)height * width * channels < ((int64_t)1 << 31),
-             "gs_l1_ssim_bwd: image %dx%dx%d too large", height, width, channels);
+             "%s: image %dx%dx%d too large", name, height, width, channels);
   const SsimLayout L = ssim_layout(height, width, channels);
-  GS_REQUIRE(workspace_bytes >= L.total, "gs_l1_ssim_bwd: workspace of %zu bytes, %zu needed", workspace_bytes,
+  GS_REQUIRE(workspace_bytes >= L.total, "%s: workspace of %zu bytes, %zu needed", name, workspace_bytes,
              L.total);
   hipStream_t s = (hipStream_t)stream;
   const float inv = (float)(1.0 / (double)L.count);
@@ -616,20 +678,37 @@ extern "C" int gs_l1_ssim_bwd(void* stream, int height, int width, int channels,
   const bool vec = whole_groups(width, pred, target, grad_pred);
   const Taps taps = make_taps();
   switch (channels) {
-    case 1: hipLaunchKernelGGL(l1_ssim_bwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
-    case 2: hipLaunchKernelGGL(l1_ssim_bwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
-    case 3: hipLaunchKernelGGL(l1_ssim_bwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
-    default: hipLaunchKernelGGL(l1_ssim_bwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, grad_out, vec, grad_pred); break;
+    case 1: hipLaunchKernelGGL(l1_ssim_bwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
+    case 2: hipLaunchKernelGGL(l1_ssim_bwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
+    case 3: hipLaunchKernelGGL(l1_ssim_bwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
+    default: hipLaunchKernelGGL(l1_ssim_bwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
   }
   GS_LAUNCH_CHECK("l1_ssim_bwd_kernel");
   return GS_OK;
+}
+}  // namespace
+
+extern "C" int gs_l1_ssim_bwd(void* stream, int height, int width, int channels, const float* pred,
+                              const float* target, const float* grad_out, const void* workspace,
+                              size_t workspace_bytes, float* grad_pred) {
+  return l1_ssim_bwd_run("gs_l1_ssim_bwd", stream, height, width, channels, pred, target, LossCot{grad_out}, workspace,
+                         workspace_bytes, grad_pred);
+}
+
+extern "C" int gs_l1_ssim_loss_bwd(void* stream, int height, int width, int channels, const float* pred,
+                                   const float* target, double lambda_ssim, const float* l1_ssim,
+                                   const float* g_total, const float* g_l1, const float* g_d_ssim,
+                                   const void* workspace, size_t workspace_bytes, float* grad_pred) {
+  const LossCot cot{nullptr, l1_ssim, g_total, g_l1, g_d_ssim, (float)lambda_ssim, (float)(1.0 - lambda_ssim)};
+  return l1_ssim_bwd_run("gs_l1_ssim_loss_bwd", stream, height, width, channels, pred, target, cot, workspace,
+                         workspace_bytes, grad_pred);
 }
 
 extern "C" int gs_l1_ssim_terms(void* stream, const float* l1_ssim, double lambda_ssim, float* terms) {
   GS_REQUIRE(l1_ssim && terms, "gs_l1_ssim_terms: NULL argument");
   GS_REQUIRE(lambda_ssim >= 0.0 && lambda_ssim <= 1.0, "gs_l1_ssim_terms: lambda must be in [0, 1]");
-  hipLaunchKernelGGL(l1_ssim_terms_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, l1_ssim, (float)lambda_ssim,
-                     (float)(1.0 - lambda_ssim), terms);
+  hipLaunchKernelGGL(l1_ssim_terms_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, l1_ssim,
+                     LossOut{(float)lambda_ssim, (float)(1.0 - lambda_ssim), terms, nullptr, nullptr, nullptr});
   GS_LAUNCH_CHECK("l1_ssim_terms_kernel");
   return GS_OK;
 }
@@ -664,7 +743,8 @@ extern "C" int gs_l1_ssim_window(void* stream, int height, int width, int channe
   hipLaunchKernelGGL(ssim_any_map_kernel, dim3(A.nblk), dim3(256), 0, s, height, width, channels, pred, target, t,
                      (const float*)V, inv, G, part);
   GS_LAUNCH_CHECK("ssim_any_map_kernel");
-  hipLaunchKernelGGL(l1_ssim_sum_kernel, dim3(1), dim3(1024), 0, s, (const float2*)part, A.nblk, inv, out);
+  hipLaunchKernelGGL(l1_ssim_sum_kernel<false>, dim3(1), dim3(1024), 0, s, (const float2*)part, A.nblk, inv, out,
+                     LossOut{});
   GS_LAUNCH_CHECK("l1_ssim_sum_kernel");
   return GS_OK;
 }

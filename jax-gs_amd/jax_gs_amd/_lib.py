@@ -104,6 +104,8 @@ _SIGS = {
     "gs_preprocess_bwd_adam": [_P, _I64, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _F, _F, _F, _F, _P, _P, _P, _I,
                                ctypes.c_double, ctypes.c_double, ctypes.c_double, _P, _P, _P, _F, _F, _P, _P, _P],
     "gs_l1_ssim_terms": [_P, _P, ctypes.c_double, _P],
+    "gs_l1_ssim_loss": [_P, _I, _I, _I, _P, _P, ctypes.c_double, _P, _P, _P, _P, _P, _I, _P, _SZ],
+    "gs_l1_ssim_loss_bwd": [_P, _I, _I, _I, _P, _P, ctypes.c_double, _P, _P, _P, _P, _P, _SZ, _P],
     "gs_adam_step": [_P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I, ctypes.c_double, ctypes.c_double,
                      ctypes.c_double],
     "gs_densify_accumulate": [_P, _I64, _P, _P, _P, _F, _F, _P, _P, _P, _P, _P, _P],

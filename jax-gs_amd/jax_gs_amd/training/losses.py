@@ -103,6 +103,42 @@ class _L1SSIM(torch.autograd.Function):
         return grad, None, None
 
 
+class _L1SSIMLoss(torch.autograd.Function):
+    """l1_ssim_loss in the launches of the means: the total, l1 and d_ssim are written by the
+    final sum, and the backward kernel forms the means' cotangents from theirs (about 25 scalar
+    torch kernels otherwise).  Window 11, at most 4 channels."""
+
+    @staticmethod
+    def forward(ctx, pred, target, lam):
+        pred = pred.contiguous()
+        target = target.contiguous()
+        H, W, C = pred.shape
+        dev = pred.device
+        nbytes = _lib.lib().gs_l1_ssim_workspace_size(H, W, C)
+        ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
+        means = torch.empty((2,), dtype=torch.float32, device=dev)
+        total, l1, d = [torch.empty((), dtype=torch.float32, device=dev) for _ in range(3)]
+        grad_needed = ctx.needs_input_grad[0]
+        _lib.call("gs_l1_ssim_loss", _lib.stream_handle(dev), H, W, C, _lib.ptr(pred), _lib.ptr(target), lam,
+                  _lib.ptr(means), None, _lib.ptr(total), _lib.ptr(l1), _lib.ptr(d), int(grad_needed), _lib.ptr(ws),
+                  nbytes)
+        ctx.set_materialize_grads(False)
+        ctx.lam = lam
+        if grad_needed:
+            ctx.save_for_backward(pred, target, ws, means)
+        return total, l1, d
+
+    @staticmethod
+    def backward(ctx, *cots):
+        pred, target, ws, means = ctx.saved_tensors
+        H, W, C = pred.shape
+        grad = torch.empty_like(pred)
+        cots = [None if g is None else g.to(device=pred.device, dtype=torch.float32).contiguous() for g in cots]
+        _lib.call("gs_l1_ssim_loss_bwd", _lib.stream_handle(pred.device), H, W, C, _lib.ptr(pred), _lib.ptr(target),
+                  ctx.lam, _lib.ptr(means), *[_lib.ptr(g) for g in cots], _lib.ptr(ws), ws.numel(), _lib.ptr(grad))
+        return grad, None, None
+
+
 def l1_and_ssim(pred: torch.Tensor, target: torch.Tensor, window_size: int = 11):
     """(mean |pred - target|, mean SSIM) of [H, W, C] images from one forward kernel;
     window_size in [1, 63] (losses.py:16)."""
@@ -134,6 +170,9 @@ def d_ssim_loss(pred: torch.Tensor, target: torch.Tensor) -> torch.Tensor:
 def l1_ssim_loss(pred: torch.Tensor, target: torch.Tensor, lambda_ssim: float = 0.2):
     """trainer.py:18-26: ((1 - lambda) l1 + lambda d_ssim, l1, d_ssim), all three from one
     forward kernel; the backward writes the image gradient of the total in one kernel."""
+    _check("ssim", pred, target)
+    if pred.dim() == 3 and pred.shape[2] <= 4 and type(lambda_ssim) in (int, float):
+        return _L1SSIMLoss.apply(pred, target, float(lambda_ssim))
     l1, s = l1_and_ssim(pred, target)
     d = _d_ssim(s)
     return (1.0 - lambda_ssim) * l1 + lambda_ssim * d, l1, d

@@ -118,16 +118,16 @@ def _train_step_fused(state, target_image, camera, optimizer, sh_degree, fast_tp
         segs = new_segments(H, W, dev)
         image, fT, nc, _ = composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg, residuals=True,
                                      clear_records=grec, window=b["window"], bins=b, segments=segs)
-        # loss (trainer.py:18-26): one kernel for the L1 and SSIM means
+        # loss (trainer.py:18-26): the L1 and SSIM means, and with their final sum d_ssim, the
+        # total and the cotangents of (l1, ssim)
         tgt = target_image.to(device=dev, dtype=torch.float32).contiguous()
         Hh, Ww, C = image.shape
         nbytes = _lib.lib().gs_l1_ssim_workspace_size(Hh, Ww, C)
         ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
         out = torch.empty((2,), dtype=torch.float32, device=dev)
-        _lib.call("gs_l1_ssim", s, Hh, Ww, C, _lib.ptr(image), _lib.ptr(tgt), _lib.ptr(out), 1, _lib.ptr(ws), nbytes)
-        # d_ssim, the total and the cotangents of (l1, ssim) in one launch
         terms = torch.empty((5,), dtype=torch.float32, device=dev)
-        _lib.call("gs_l1_ssim_terms", s, _lib.ptr(out), float(lambda_ssim), _lib.ptr(terms))
+        _lib.call("gs_l1_ssim_loss", s, Hh, Ww, C, _lib.ptr(image), _lib.ptr(tgt), float(lambda_ssim), _lib.ptr(out),
+                  _lib.ptr(terms), None, None, None, 1, _lib.ptr(ws), nbytes)
         l1, total, gout = out[0], terms[1], terms[2:4]
         gimg = torch.empty_like(image)
         _lib.call("gs_l1_ssim_bwd", s, Hh, Ww, C, _lib.ptr(image), _lib.ptr(tgt), _lib.ptr(gout), _lib.ptr(ws), nbytes,

@@ -47,3 +47,46 @@ def test_l1_ssim_tile_edges(cuda, H, W, C, shift):
     want = 0.8 * seed.astype(np.float64) + oracle.ssim_vjp(pred, tgt, -0.1)
     got = g[shift:shift + count].reshape(shape)
     assert np.linalg.norm(got - want) <= 1e-4 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("which", [(1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)])
+@pytest.mark.parametrize("lam", [0.2, 0.0, 1])
+def test_l1_ssim_loss_and_cotangents(cuda, lam, which):
+    """l1_ssim_loss's three outputs and the gradient from any of their cotangents against the
+    composition of l1_and_ssim: the outputs' bits, the gradient to float32 rounding of its two
+    scalar cotangents."""
+    from jax_gs_amd.training import losses
+
+    rng = np.random.default_rng(3)
+    t = torch.from_numpy(rng.uniform(0, 1, (21, 130, 3)).astype(np.float32)).to(cuda)
+    p0 = (t + 0.1 * torch.from_numpy(rng.normal(0, 1, t.shape).astype(np.float32)).to(cuda)).clamp(0, 1)
+    outs, grads = [], []
+    for fused in (True, False):
+        p = p0.clone().requires_grad_(True)
+        if fused:
+            o = losses.l1_ssim_loss(p, t, lam)
+        else:
+            l1, s = losses.l1_and_ssim(p, t)
+            d = losses._d_ssim(s)
+            o = ((1.0 - lam) * l1 + lam * d, l1, d)
+        sum(w * (k + 1.5) * v for k, (w, v) in enumerate(zip(which, o)) if w).backward()
+        outs.append([float(v.detach()) for v in o])
+        grads.append(p.grad)
+    assert outs[0] == outs[1]
+    scale = grads[1].norm()
+    assert (grads[0] - grads[1]).norm() <= 1e-6 * scale if scale > 0 else not grads[0].any()
+
+
+def test_l1_ssim_loss_of_equal_images(cuda):
+    """At SSIM = 1 the max ties or rounds: the gradient follows torch.maximum's half."""
+    from jax_gs_amd.training import losses
+
+    t = torch.rand((40, 50, 3), device=cuda)
+    grads = []
+    for fused in (True, False):
+        p = t.clone().requires_grad_(True)
+        l1, s = (None, None) if fused else losses.l1_and_ssim(p, t)
+        total = losses.l1_ssim_loss(p, t)[0] if fused else 0.8 * l1 + 0.2 * losses._d_ssim(s)
+        total.backward()
+        grads.append(p.grad)
+    assert (grads[0] - grads[1]).norm() <= 1e-6 * grads[1].norm() + 1e-12
