@@ -1539,20 +1539,33 @@ __global__ void zero_grads_kernel(float4* __restrict__ p, int64_t n4, float* __r
 }
 
 // dL/dbackground = sum over pixels of T_final * g (rasterizer.py:244): grid-stride
-// partial sums, a block reduction and 3 atomics per block.
+// partial sums (four pixels in flight per lane), a block reduction and 3 atomics per block.  The
+// atomics meet at three addresses, one after another: with 1024 blocks they took most of the
+// launch's 15.4 us at 640x479 (18.8 at 1920x1080); 2048 pixels a block, at most 256 blocks.
 __global__ __launch_bounds__(256) void background_grad_kernel(int64_t npix, int W, int H,
                                                               const float* __restrict__ finalT, const ImageCot gc,
                                                               float* __restrict__ gbg) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const float sc = l1_scale(gc, W, H);
   float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < npix; p += stride) {
-    const float t = finalT[p];
-    float g0, g1, g2;
-    image_cot(gc, sc, p, g0, g1, g2);
-    a0 = fmaf(t, g0, a0);
-    a1 = fmaf(t, g1, a1);
-    a2 = fmaf(t, g2, a2);
+  for (int64_t p0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p0 < npix; p0 += 4 * stride) {
+    float t[4], g[4][3];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t p = p0 + u * stride;
+      t[u] = 0.0f;
+      g[u][0] = g[u][1] = g[u][2] = 0.0f;
+      if (p < npix) {
+        t[u] = finalT[p];
+        image_cot(gc, sc, p, g[u][0], g[u][1], g[u][2]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a0 = fmaf(t[u], g[u][0], a0);
+      a1 = fmaf(t[u], g[u][1], a1);
+      a2 = fmaf(t[u], g[u][2], a2);
+    }
   }
   a0 = wave_sum(a0);
   a1 = wave_sum(a1);
@@ -1993,7 +2006,7 @@ int composite_bwd_run(const char* name, void* stream, int64_t n, const float* re
   }
   if (grad_background) {
     const int64_t npix = (int64_t)width * height;
-    hipLaunchKernelGGL(background_grad_kernel, dim3(std::min<int64_t>(1024, div_up(npix, 256))), dim3(256), 0, s,
+    hipLaunchKernelGGL(background_grad_kernel, dim3(std::min<int64_t>(256, div_up(npix, 2048))), dim3(256), 0, s,
                        npix, width, height, final_T, gc, grad_background);
     GS_LAUNCH_CHECK("background_grad_kernel");
   }
