@@ -1116,8 +1116,9 @@ __global__ __launch_bounds__(kWinThreads) void window_bins_kernel(
 // contiguous run per store.  Lane u holds tile u's next slot (read with v_readlane,
 // advanced once per step).  A chunk costs two memory round trips: its descriptor
 // (with its counts), then its 256 words and the tiles' range starts together.
-// CHECK: some entries fall beyond the capacity and are dropped.
-template <bool WITH_TILES, bool CHECK>
+// CHECK: some entries fall beyond the capacity and are dropped.  STORE: false advances the slots
+// past the step and writes nothing.
+template <bool WITH_TILES, bool CHECK, bool STORE>
 __device__ inline void write_step(uint64_t word, bool act, int sx, int sy, int lane, uint32_t n_gauss, int TX,
                                   uint32_t cap32, uint32_t& base, int32_t* __restrict__ out_gid,
                                   int32_t* __restrict__ out_tile) {
@@ -1132,7 +1133,7 @@ __device__ inline void write_step(uint64_t word, bool act, int sx, int sy, int l
     rm[k] = __ballot(act && g.y0 <= ty && ty < g.y0 + g.h);
   }
 #pragma unroll
-  for (int uy = 0; uy < kSB; ++uy) {
+  for (int uy = 0; STORE && uy < kSB; ++uy) {
     if (rm[uy] == 0ull) continue;
 #pragma unroll
     for (int ux = 0; ux < kSB; ++ux) {
@@ -1161,10 +1162,17 @@ __device__ inline void write_step(uint64_t word, bool act, int sx, int sy, int l
   base += (uint32_t)__popcll(mine & rmine);
 }
 
+// Up to this many chunks a chunk's four steps go to four waves (tile_write_kernel): 16k Gaussians
+// at 256x256 16.6 -> 9.5 us, 50k at 640x479 (about 300 chunks) 17.9 -> 11.1; at about 2000 chunks
+// (400k) the GPU is full without it and each wave's reads and slots of the earlier steps cost more
+// than they save: 20.2 -> 21.1.
+constexpr uint32_t kSplitChunks = 1024;
+
+// Steps s0 .. s1 - 1 of a chunk.
 template <bool WITH_TILES, bool CHECK>
 __device__ inline void write_chunk(const uint4& d, const uint64_t* __restrict__ pval, uint32_t n_gauss, int TX, int TY,
                                    uint32_t cnt_c, const uint32_t* __restrict__ seg_pre,
-                                   const int32_t* __restrict__ ranges, uint32_t cap32, int lane,
+                                   const int32_t* __restrict__ ranges, uint32_t cap32, int lane, int s0, int s1,
                                    int32_t* __restrict__ out_gid, int32_t* __restrict__ out_tile) {
   const int len = (int)(d.y & 0xFFFFu), sx = (int)(d.z & 0xFFFFu), sy = (int)(d.z >> 16);
   const int t = tile_of(sx, sy, lane, TX, TY);
@@ -1174,11 +1182,17 @@ __device__ inline void write_chunk(const uint4& d, const uint64_t* __restrict__ 
   // lane u: next slot of tile u (tiles outside the image never get entries): the
   // tile's range start + the superblock's earlier segments + earlier chunks of this one
   uint32_t base = (t >= 0 ? (uint32_t)ranges[t] : 0u) + seg_pre[(int64_t)d.w * 64 + lane] + cnt_c;
+  // the steps before the wave's own only move the slots
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-    if (64 * k < len)
-      write_step<WITH_TILES, CHECK>(wv[k], 64 * k + lane < len, sx, sy, lane, n_gauss, TX, cap32, base, out_gid,
-                                    out_tile);
+  for (int k = 0; k < 4; ++k) {
+    if (64 * k >= len || k >= s1) continue;
+    if (k < s0)
+      write_step<WITH_TILES, CHECK, false>(wv[k], 64 * k + lane < len, sx, sy, lane, n_gauss, TX, cap32, base, out_gid,
+                                           out_tile);
+    else
+      write_step<WITH_TILES, CHECK, true>(wv[k], 64 * k + lane < len, sx, sy, lane, n_gauss, TX, cap32, base, out_gid,
+                                          out_tile);
+  }
 }
 
 // The default path's chunk window of the list being written (NULL win: none), with the
@@ -1234,7 +1248,13 @@ __global__ __launch_bounds__(256) void tile_write_kernel(const uint32_t* __restr
   const uint32_t cap32 = (uint32_t)cap;  // gs_bin checks cap < 2^31
   // every entry fits (the usual case): no per-store capacity test
   const bool fits = ranges[T] >= 0 && (int64_t)ranges[T] <= cap;
-  for (uint32_t c = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); c < C; c += nwaves) {
+  // A step stores up to 64 runs one after another; where chunks are fewer than waves the launch
+  // is one chunk's four steps long, so four waves take a step each (kSplitChunks).
+  const bool split = C <= kSplitChunks;
+  const uint32_t items = split ? 4 * C : C;
+  for (uint32_t it = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); it < items; it += nwaves) {
+    const uint32_t c = split ? it >> 2 : it;
+    const int s0 = split ? __builtin_amdgcn_readfirstlane((int)(it & 3u)) : 0, s1 = split ? s0 + 1 : 4;
     const uint4 d = desc[c];
     // counts of the chunk's earlier chunks in its segment (p of them), loaded together
     const uint32_t p = d.y >> 16;
@@ -1242,9 +1262,11 @@ __global__ __launch_bounds__(256) void tile_write_kernel(const uint32_t* __restr
 #pragma unroll
     for (int k = 1; k < kSeg; ++k) cnt_c += (uint32_t)k <= p ? cnt[(int64_t)(c - k) * 64 + lane] : 0u;
     if (fits)
-      write_chunk<WITH_TILES, false>(d, pval, n_gauss, TX, TY, cnt_c, seg_pre, ranges, cap32, lane, out_gid, out_tile);
+      write_chunk<WITH_TILES, false>(d, pval, n_gauss, TX, TY, cnt_c, seg_pre, ranges, cap32, lane, s0, s1, out_gid,
+                                     out_tile);
     else
-      write_chunk<WITH_TILES, true>(d, pval, n_gauss, TX, TY, cnt_c, seg_pre, ranges, cap32, lane, out_gid, out_tile);
+      write_chunk<WITH_TILES, true>(d, pval, n_gauss, TX, TY, cnt_c, seg_pre, ranges, cap32, lane, s0, s1, out_gid,
+                                    out_tile);
   }
   if constexpr (!OFFSET) {
     if (clamped) {  // (uniform: every workgroup takes this branch or none)
