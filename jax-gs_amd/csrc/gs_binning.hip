@@ -1163,7 +1163,7 @@ __device__ inline void write_step(uint64_t word, bool act, int sx, int sy, int l
 }
 
 // Up to this many chunks a chunk's four steps go to four waves (tile_write_kernel): 16k Gaussians
-// at 256x256 16.6 -> 9.5 us, 50k at 640x479 (about 300 chunks) 17.9 -> 11.1; at about 2000 chunks
+// at 256x256 16.6 -> 9.5 us, 50k at 640x479 17.9 -> 11.1, 200k at 504x378 18.2 -> 13.0; at about 2000 chunks
 // (400k) the GPU is full without it and each wave's reads and slots of the earlier steps cost more
 // than they save: 20.2 -> 21.1.
 constexpr uint32_t kSplitChunks = 1024;
