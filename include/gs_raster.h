@@ -488,8 +488,8 @@ int gs_l1_ssim_window_bwd(void* stream, int height, int width, int channels, int
 int gs_l1_ssim_terms(void* stream, const float* l1_ssim, double lambda_ssim, float* terms);
 
 /* gs_l1_ssim and the trainer's loss from its means in the same launches: l1_ssim[2] as gs_l1_ssim's
- * out, terms[5] as gs_l1_ssim_terms, and the total, the L1 mean and d_ssim as scalars of their own
- * (each of these four may be NULL).  Any lambda. */
+ * out, terms[5] as gs_l1_ssim_terms (lambda in [0, 1] then, as there), and the total, the L1 mean
+ * and d_ssim as scalars of their own (each of these four may be NULL; any lambda without terms). */
 int gs_l1_ssim_loss(void* stream, int height, int width, int channels, const float* pred, const float* target,
                     double lambda_ssim, float* l1_ssim, float* terms, float* total, float* l1, float* d_ssim,
                     int with_grad, void* workspace, size_t workspace_bytes);

@@ -655,6 +655,8 @@ extern "C" int gs_l1_ssim(void* stream, int height, int width, int channels, con
 extern "C" int gs_l1_ssim_loss(void* stream, int height, int width, int channels, const float* pred,
                                const float* target, double lambda_ssim, float* l1_ssim, float* terms, float* total,
                                float* l1, float* d_ssim, int with_grad, void* workspace, size_t workspace_bytes) {
+  GS_REQUIRE(terms == nullptr || (lambda_ssim >= 0.0 && lambda_ssim <= 1.0),
+             "gs_l1_ssim_loss: lambda must be in [0, 1] for terms");
   const LossOut loss{(float)lambda_ssim, (float)(1.0 - lambda_ssim), terms, total, l1, d_ssim};
   return l1_ssim_fwd_run("gs_l1_ssim_loss", stream, height, width, channels, pred, target, l1_ssim, with_grad,
                          workspace, workspace_bytes, &loss);

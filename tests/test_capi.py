@@ -130,6 +130,22 @@ def test_argument_errors_of_the_fused_l1_loss():
     assert rc == 1 and b"image cotangent" in L.gs_last_error()
 
 
+@pytest.mark.parametrize("lam", [-0.01, 1.01, float("nan")])
+def test_training_loss_rejects_a_lambda_outside_0_1(lam):
+    """gs_l1_ssim_loss with terms (the training step's loss) takes the lambdas gs_l1_ssim_terms
+    takes; without them any (the next check, of the workspace, is reached)."""
+    L = _lib.lib()
+    fake = ctypes.c_void_p(256)
+    head = (None, 8, 8, 3, fake, fake)
+    assert L.gs_l1_ssim_terms(None, fake, lam, fake) == 1 and b"lambda" in L.gs_last_error()
+    assert L.gs_l1_ssim_loss(*head, lam, fake, fake, None, None, None, 1, fake, 0) == 1
+    assert b"lambda" in L.gs_last_error()
+    assert L.gs_l1_ssim_loss(*head, lam, fake, None, fake, fake, fake, 1, fake, 0) == 1
+    assert b"workspace" in L.gs_last_error()
+    assert L.gs_l1_ssim_loss(*head, 0.2, fake, fake, None, None, None, 1, fake, 0) == 1
+    assert b"workspace" in L.gs_last_error()
+
+
 def test_clear_list_and_zeroed_arguments():
     """gs_composite_bwd rejects a clear list with a negative count or a NULL array with a
     count, before launching anything; clear_list() builds the gs_clear_list_t layout."""
