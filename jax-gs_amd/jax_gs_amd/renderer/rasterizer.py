@@ -241,17 +241,18 @@ class _RenderTiles(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, means2D, cov2D, opacities, colors, bg, gids, ranges, win, static):
-        H, W = static
+        H, W, grad = static  # needs_input_grad is set under torch.no_grad() too
         rec = composite_records(means2D, cov2D, opacities, colors)
-        segs = new_segments(H, W, rec.device) if any(ctx.needs_input_grad[:5]) else None
-        image, fT, nc, _ = composite(rec, gids, ranges, H, W, bg, residuals=True, window=win, segments=segs)
+        segs = new_segments(H, W, rec.device) if grad and any(ctx.needs_input_grad[:5]) else None
+        image, fT, nc, _ = composite(rec, gids, ranges, H, W, bg, residuals=segs is not None, window=win,
+                                     segments=segs)
         ctx.static = static
         ctx.save_for_backward(cov2D, opacities, bg, rec, gids, ranges, win, fT, nc, segs)
         return image
 
     @staticmethod
     def backward(ctx, g_image):
-        H, W = ctx.static
+        H, W, _ = ctx.static
         cov2D, opacities, bg, rec, gids, ranges, win, fT, nc, segs = ctx.saved_tensors
         dev = rec.device
         n = rec.shape[0]
@@ -286,7 +287,8 @@ def _render_tiles(means2D, cov2D, opacities, colors, sorted_tile_ids, sorted_gau
     bg = background_tensor(background, dev)
     gids = sorted_gaussian_ids.to(torch.int32).contiguous()
     win = window_from_list(gids) if clamped_windows else None
-    return _RenderTiles.apply(m, c, o, col, bg, gids, ranges, win, (int(H), int(W)))
+    return _RenderTiles.apply(m, c, o, col, bg, gids, ranges, win,
+                              (int(H), int(W), torch.is_grad_enabled()))
 
 
 def render_tiles(means2D, cov2D, opacities, colors, sorted_tile_ids, sorted_gaussian_ids, H, W,
