@@ -90,8 +90,8 @@ const char* gs_last_error(void);
  * builds it; gs_window_from_bins stays for lists binned without it).  14: gs_composite_bwd
  * and gs_composite_bwd_l1 take a gs_clear_list_t; gs_preprocess_bwd and
  * gs_preprocess_bwd_w2c take zeroed.  Added since, with every call of 14 as it was:
- * gs_composite_segments_size, gs_composite_fwd_seg, gs_composite_bwd_seg; gs_l1_ssim_loss,
- * gs_l1_ssim_loss_bwd. */
+ * gs_composite_segments_size, gs_composite_segments_size_for, gs_composite_fwd_seg,
+ * gs_composite_bwd_seg; gs_l1_ssim_loss, gs_l1_ssim_loss_bwd. */
 int gs_abi_version(void);
 
 /* Projection + covariance + SH colour for every Gaussian.
@@ -327,8 +327,13 @@ int gs_composite_bwd_l1(void* stream, int64_t n, const float* records, const int
  * in several waves at once (a tile's walk is a serial chain; the longest one was most
  * launches' time).  Replaces the same reference code as gs_composite_fwd and gs_composite_bwd.
  *
- * gs_composite_segments_size: bytes of the segments array (16-byte aligned) that the forward
- *   writes and the backward of the same render reads.
+ * gs_composite_segments_size_for: bytes of the segments array (16-byte aligned) that the forward
+ *   with this capacity writes and the backward of the same render reads: 4 bytes per tile from
+ *   6144 tiles on; below, 4 KB for each segment that lists of `capacity` entries can have, T +
+ *   capacity / 128 (T tiles, from 2048 on) or T + capacity / 64 (fewer), and at most 16 (64 KB)
+ *   or 32 (128 KB) per tile: 101 MB at 504x378, 142 at 979x546, 236 at 1280x720, 401 at
+ *   1440x1079.
+ * gs_composite_segments_size: that most, enough for lists of any length.
  * gs_composite_fwd_seg: gs_composite_fwd (stats and bin_workspace NULL; capacity = the list's
  *   length) or gs_composite_fwd_deferred (both given), with segments in tile_order's place;
  *   l1_target and l1_out (NULL, or both as in gs_composite_fwd_deferred_l1) fuse the L1 loss.
@@ -336,6 +341,7 @@ int gs_composite_bwd_l1(void* stream, int64_t n, const float* records, const int
  *   gs_composite_bwd_l1 (grad_image may then be NULL), with that segments array in
  *   tile_order's place.  The gradients are the same sums: the transmittance and the colour
  *   behind a segment's last entry come from the forward instead of the entries behind it. */
+size_t gs_composite_segments_size_for(int width, int height, int64_t capacity);
 size_t gs_composite_segments_size(int width, int height);
 int gs_composite_fwd_seg(void* stream, int64_t n, const float* records, int32_t* sorted_gids, int64_t capacity,
                          const int32_t* ranges, const int32_t* stats, const void* bin_workspace,

@@ -46,6 +46,7 @@
 #include "gs_bins.h"
 #include "gs_common.h"
 #include "gs_cull.h"
+#include "gs_segments.h"
 
 #include <algorithm>
 
@@ -438,60 +439,6 @@ __device__ inline void clear_share(float4* __restrict__ clear, int64_t n_clear) 
   }
 }
 
-constexpr int kQuadTiles = 2048;  // images below are composited by composite_fwd_quad_kernel
-
-// Segments of a tile's list.  The backward walks a tile's entries back to front, a serial
-// chain like the forward's, and the longest tile's chain was most launches' time (2170 tiles
-// of 274 entries on average: the one of 1046 took 283 us while the work of all would fill the
-// GPU for 50).  The forward therefore cuts every list into segments, 1024/u of u entries, then
-// 512/u of 2u and 512/u of 4u (4096 in all; log2 u = segment_shift), and leaves for each segment it
-// completes, per pixel, the transmittance after it and the colour blended in it.  The backward
-// then walks all segments at once: a segment starts from its own end's transmittance, and the
-// colour behind it is the background's share plus the later segments' colours, summed from
-// the back, so neither is recovered through the entries behind it.
-// Backward, whole lists -> segments: 300k Gaussians at 979x546 283 -> 95 us, 200k at 504x378
-// 217 -> 75, 50k at 640x479 170 -> 66, 2k at 96x64 90 -> 22, 2.1M at 1280x720 284 -> 197 (which
-// zeroes 500 MB besides); the order of the items instead of the tiles' 4.8 -> 10 us, the slots
-// add 5-8 us to the forward.
-// Slot j of a tile (256 pixels, row by row): (T after segment j, colour r g b of segment j).
-// A pixel's slots are written for every segment it enters, except where its wave never leaves
-// segment 0 (there the final T and the background say it all).
-// The backward's work items are pieces: the segments of a coarser unit, the smallest of u, 2u,
-// .. 512 at which the pieces of all tiles fit the launch's grid (segment_grid; every coarser
-// unit's ends are ends of segments of u, and at 512 a tile has at most four).
-struct Segments {
-  int32_t* items;   // [0] = number of pieces, [1] = log2 of their unit, then tile * 32 + piece, longest first
-  int32_t* met;     // per tile, the entries met by each of the forward's waves
-  float4* slots;    // [T][segment_count(u)][256]; NULL: the forward leaves none
-  int lu;           // log2(u)
-};
-// From kFwdOneWaveTiles tiles on, one wave per tile fills the GPU several times over, and the
-// slots' traffic and the pieces' set-up cost more than they balance (8160 tiles, the longest
-// of 781 entries: backward 247 -> 255 us, its order 8 -> 13 us): no segments there.
-constexpr int kFwdOneWaveTiles = 6 * 1024;
-// Units: 64 entries where tiles are few (200k Gaussians, 504x378: 128 91 us, 64 75), 128 where
-// they fill the GPU sooner and a piece's set-up has to be earned back (300k, 979x546: 64 99 us,
-// 128 95, 256 121).
-__host__ __device__ inline int segment_shift(int T) { return T < kQuadTiles ? 6 : 7; }  // log2(u)
-__host__ __device__ inline int segment_count(int lu) { return 2048 >> lu; }
-__host__ __device__ inline int segment_start(int j, int lu) {
-  const int n0 = 1024 >> lu, n1 = n0 + (n0 >> 1);
-  return j <= n0 ? j << lu : (j <= n1 ? 1024 + ((j - n0) << (lu + 1)) : 2048 + ((j - n1) << (lu + 2)));
-}
-// segments that hold the first k entries (k <= 4096)
-__host__ __device__ inline int segments_within(int k, int lu) {
-  const int n0 = 1024 >> lu, n1 = n0 + (n0 >> 1);
-  const int up = (1 << lu) - 1, up1 = (2 << lu) - 1, up2 = (4 << lu) - 1;
-  return k <= 1024 ? (k + up) >> lu : (k <= 2048 ? n0 + ((k - 1024 + up1) >> (lu + 1)) : n1 + ((k - 2048 + up2) >> (lu + 2)));
-}
-// Most pieces a launch takes.  Workgroups past the pieces' number exit at once, but each
-// still costs its dispatch (3600 tiles with room for 16 pieces each, 57,600 workgroups of which
-// 10,000 had work: 232 us against 203).
-__host__ __device__ inline int segment_grid(int T) {
-  const int all = T * segment_count(segment_shift(T)), some = 4 * T + 2048;
-  return all < some ? all : some;
-}
-
 // The forward of small images (below 2048 tiles).  A tile's walk is a serial chain, and the
 // longest tile's chain is the launch's time: with one pixel per lane and four waves per tile
 // an entry cost such a wave 185 cycles (16k Gaussians, 256x256, longest tile 1144 entries:
@@ -633,7 +580,7 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
     c1 = quad_sum(c1);
     c2 = quad_sum(c2);
     if (sg.slots != nullptr && e == 0)
-      sg.slots[((int64_t)tile * segment_count(sg.lu) + seg) * 256 + (yl + (lane >> 4)) * kTile + xl +
+      sg.slots[(segment_slot(sg.packed, tile, start, sg.lu) + seg) * 256 + (yl + (lane >> 4)) * kTile + xl +
                ((lane >> 2) & 3)] = make_float4(Tnow, c0, c1, c2);
   };
   for (int b0 = 0; b0 < n && open != 0ull; b0 += 64) {
@@ -763,7 +710,7 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
       if (sg.slots != nullptr)
-        sg.slots[((int64_t)tile * segment_count(sg.lu) + seg) * 256 + (part * 4 * PPT + (lane >> 4) + 4 * i) * kTile +
+        sg.slots[(segment_slot(sg.packed, tile, start, sg.lu) + seg) * 256 + (part * 4 * PPT + (lane >> 4) + 4 * i) * kTile +
                  (lane & 15)] = make_float4(Tr[i], c0[i], c1[i], c2[i]);
       if (seg > 0) {
         c0[i] += s_col[3 * i][lane];
@@ -1159,7 +1106,7 @@ __device__ __forceinline__ void composite_bwd_body(
     const ImageCot gc, const float* __restrict__ finalT, const int32_t* __restrict__ ncontrib,
     float* __restrict__ grec, const gs_window_t* __restrict__ win, const Segments sg, int tile, int piece, int part) {
   // the entries to walk: a piece of the list, or all of it
-  const int lp = SEG ? sg.items[1] : 0;
+  const int word = SEG ? sg.items[1] : 0, lp = word & 255;
   const int lo = SEG ? segment_start(piece, lp) : 0, hi = SEG ? segment_start(piece + 1, lp) : kMaxTileEntries;
   const int last = SEG ? segments_within(hi, sg.lu) - 1 : 0;  // the piece's last segment
   const int lane = threadIdx.x;
@@ -1196,7 +1143,7 @@ __device__ __forceinline__ void composite_bwd_body(
         // behind the piece's last entry: the background and the later segments' colours,
         // farthest first, over the transmittance there
         const float4* slot =
-            sg.slots + (int64_t)tile * segment_count(sg.lu) * 256 + (part * 4 * PPT + (lane >> 4) + 4 * i) * kTile + (lane & 15);
+            sg.slots + segment_slot(word >> 8, tile, start, sg.lu) * 256 + (part * 4 * PPT + (lane >> 4) + 4 * i) * kTile + (lane & 15);
         float R = Tq * Rg[i];
         for (int j = segments_within(k, sg.lu) - 1; j > last; --j) {
           const float4 d = slot[j * 256];
@@ -1783,7 +1730,7 @@ __global__ __launch_bounds__(1024) void segment_items_kernel(const Segments sg, 
   }
   if (tid == 0) {
     sg.items[0] = base;
-    sg.items[1] = lp;
+    sg.items[1] = lp + (sg.packed ? 256 : 0);
   }
 #pragma unroll
   for (int i = 0; i < kPer; ++i)
@@ -1838,21 +1785,22 @@ extern "C" int gs_window_from_list(void* stream, const int32_t* sorted_gids, int
 namespace {
 // A segments buffer: the items, the waves' met counts, the slots; from kFwdOneWaveTiles tiles
 // on, where lists have no segments, the tile order.
-int64_t segments_layout(int T, int64_t* met, int64_t* slots) {
+int64_t segments_layout(int T, int64_t capacity, int64_t* met, int64_t* slots) {
   if (T >= kFwdOneWaveTiles) return (int64_t)T * 4;
   auto up = [](int64_t b) { return (b + 255) & ~(int64_t)255; };
   *met = up(4 * (2 + (int64_t)segment_grid(T)));
   *slots = *met + up((int64_t)T * (T < kQuadTiles ? kQuadParts : 2) * 4);
-  return *slots + (int64_t)T * segment_count(segment_shift(T)) * 256 * (int64_t)sizeof(float4);
+  return *slots + segment_slots(T, capacity, segment_shift(T)) * 256 * (int64_t)sizeof(float4);
 }
-Segments segments_of(void* p, int T) {
-  Segments sg{nullptr, nullptr, nullptr, segment_shift(T)};
+Segments segments_of(void* p, int T, int64_t capacity) {
+  Segments sg{nullptr, nullptr, nullptr, segment_shift(T), false};
   if (p != nullptr) {
     int64_t met, slots;
-    segments_layout(T, &met, &slots);
+    segments_layout(T, capacity, &met, &slots);
     sg.items = (int32_t*)p;
     sg.met = (int32_t*)((char*)p + met);
     sg.slots = (float4*)((char*)p + slots);
+    sg.packed = segments_packed(T, capacity, sg.lu);
   }
   return sg;
 }
@@ -1889,7 +1837,7 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
     tile_order = (int32_t*)segments;
     segments = nullptr;
   }
-  const Segments sg = segments_of(segments, T);
+  const Segments sg = segments_of(segments, T, n_entries);
 #define GS_FWD_LAUNCH2(PPT, WPT, WIN, O32, SB)                                                                  \
   hipLaunchKernelGGL((composite_fwd_kernel<PPT, WIN, O32, SB>), dim3(nblk * (WPT)), dim3(64), 0, s,             \
                      (const float4*)records, (int)n, sorted_gids, n_entries, ranges, width, height, TX, T,        \
@@ -2021,7 +1969,7 @@ int composite_bwd_run(const char* name, void* stream, int64_t n, const float* re
     tile_order = (const int32_t*)segments;
     segments = nullptr;
   }
-  const Segments sg = segments_of(const_cast<void*>(segments), T);
+  const Segments sg = segments_of(const_cast<void*>(segments), T, n_entries);
   const int nblk = segments ? segment_grid(T) : tile_blocks(TX, TY);
 #define GS_BWD_LAUNCH(KERNEL, WPT)                                                                                  \
   hipLaunchKernelGGL(KERNEL, dim3(nblk * (WPT)), dim3(64), 0, s, (const float4*)records, (int)n, sorted_gids, n_entries, \
@@ -2076,10 +2024,14 @@ extern "C" int gs_composite_bwd_l1(void* stream, int64_t n, const float* records
                            accumulate, window, clear);
 }
 
-extern "C" size_t gs_composite_segments_size(int width, int height) {
-  if (width <= 0 || height <= 0) return 0;
+extern "C" size_t gs_composite_segments_size_for(int width, int height, int64_t capacity) {
+  if (width <= 0 || height <= 0 || capacity < 0) return 0;
   int64_t met, slots;
-  return (size_t)segments_layout(((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile), &met, &slots);
+  return (size_t)segments_layout(((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile), capacity, &met, &slots);
+}
+
+extern "C" size_t gs_composite_segments_size(int width, int height) {
+  return gs_composite_segments_size_for(width, height, INT64_MAX >> 8);
 }
 
 extern "C" int gs_composite_fwd_seg(void* stream, int64_t n, const float* records, int32_t* sorted_gids,

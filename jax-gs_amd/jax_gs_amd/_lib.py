@@ -73,6 +73,7 @@ _SIGS = {
     "gs_composite_bwd_l1": [_P, _I64, _P, _P, _I64, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P,
                             _P],
     "gs_composite_segments_size": [_I, _I],
+    "gs_composite_segments_size_for": [_I, _I, _I64],
     "gs_composite_fwd_seg": [_P, _I64, _P, _P, _I64, _P, _P, _P, _SZ, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P],
     "gs_composite_bwd_seg": [_P, _I64, _P, _P, _I64, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P,
                              _P],
@@ -114,7 +115,8 @@ _RESTYPE = {"gs_last_error": ctypes.c_char_p, "gs_bin_workspace_size": _SZ, "gs_
             "gs_bin_deferred_workspace_size": _SZ,
             "gs_bin_reference_workspace_size": _SZ, "gs_preprocess_bwd_w2c_workspace_size": _SZ,
             "gs_l1_ssim_window_workspace_size": _SZ,
-            "gs_densify_workspace_size": _SZ, "gs_composite_segments_size": _SZ, "gs_composite_l1_out_size": _I64}
+            "gs_densify_workspace_size": _SZ, "gs_composite_segments_size": _SZ,
+            "gs_composite_segments_size_for": _SZ, "gs_composite_l1_out_size": _I64}
 
 _lib = None
 

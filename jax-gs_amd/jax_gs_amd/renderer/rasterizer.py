@@ -151,9 +151,13 @@ def composite_records(means2D, cov2D, opacities, colors) -> torch.Tensor:
     return rec
 
 
-def new_segments(H: int, W: int, dev) -> torch.Tensor:
-    """Storage for the segments that a compositing forward leaves to its backward."""
-    return torch.empty((_lib.lib().gs_composite_segments_size(int(W), int(H)),), dtype=torch.uint8, device=dev)
+def new_segments(H: int, W: int, dev, capacity: int | None = None) -> torch.Tensor:
+    """Storage for the segments that a compositing forward over a list of `capacity` entries
+    (its length) leaves to its backward; None: lists of any length.  Below 6144 tiles 4 KB per
+    segment, held until the backward: at most 64 or 128 KB per tile (142 MB at 979x546)."""
+    size = (_lib.lib().gs_composite_segments_size(int(W), int(H)) if capacity is None
+            else _lib.lib().gs_composite_segments_size_for(int(W), int(H), int(capacity)))
+    return torch.empty((size,), dtype=torch.uint8, device=dev)
 
 
 def _check_bins(bins: BinResult, records, sorted_gids, ranges) -> None:
@@ -243,7 +247,7 @@ class _RenderTiles(torch.autograd.Function):
     def forward(ctx, means2D, cov2D, opacities, colors, bg, gids, ranges, win, static):
         H, W, grad = static  # needs_input_grad is set under torch.no_grad() too
         rec = composite_records(means2D, cov2D, opacities, colors)
-        segs = new_segments(H, W, rec.device) if grad and any(ctx.needs_input_grad[:5]) else None
+        segs = new_segments(H, W, rec.device, gids.shape[0]) if grad and any(ctx.needs_input_grad[:5]) else None
         image, fT, nc, _ = composite(rec, gids, ranges, H, W, bg, residuals=segs is not None, window=win,
                                      segments=segs)
         ctx.static = static

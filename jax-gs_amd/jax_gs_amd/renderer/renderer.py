@@ -48,7 +48,7 @@ def _render_forward(ctx, means, scales, quats, opac, sh, w2c, bg, mask, static, 
             if grad and any(ctx.needs_input_grad[:5]) else None)
     win = b["window"]
     # the lists' segments, which the backward walks side by side
-    segs = new_segments(H, W, means.device) if grad and any(ctx.needs_input_grad) else None
+    segs = (new_segments(H, W, means.device, b["capacity"]) if grad and any(ctx.needs_input_grad) else None)
     out = composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg, residuals=segs is not None,
                     clear_records=grec, window=win, bins=b, l1_target=target, segments=segs)
     image, fT, nc = out[:3]

@@ -115,7 +115,7 @@ def _train_step_fused(state, target_image, camera, optimizer, sh_degree, fast_tp
                           window=not fast_tpu_rasterizer, deferred=True)
         bg = background_tensor(None, dev)
         grec = torch.empty((n, _lib.GS_REC_STRIDE), dtype=torch.float32, device=dev)  # cleared by the forward
-        segs = new_segments(H, W, dev)
+        segs = new_segments(H, W, dev, b["capacity"])
         image, fT, nc, _ = composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg, residuals=True,
                                      clear_records=grec, window=b["window"], bins=b, segments=segs)
         # loss (trainer.py:18-26): the L1 and SSIM means, and with their final sum d_ssim, the

@@ -1,8 +1,11 @@
-"""What the compositing forward's segments hold: nothing where no backward can follow."""
+"""What the compositing forward's segments hold: nothing where no backward can follow, and no more
+than the list's capacity asks for."""
 import numpy as np
 import pytest
 import torch
 
+from gpu_helpers import np_, rel
+from jax_gs_amd import _lib, render, scenes
 from jax_gs_amd.renderer import rasterizer, rasterizer_tpu
 
 pytestmark = pytest.mark.gpu
@@ -39,3 +42,64 @@ def test_render_tiles_without_grad_mode_leaves_no_segments(cuda, entry):
     torch.cuda.synchronize()
     assert torch.cuda.max_memory_allocated() - before < segments / 4
     assert torch.equal(shown, image.detach())
+
+
+# tiles wide, tiles high, entries per tile (cycled): units of 64 (below 2048 tiles) and 128 entries
+@pytest.mark.parametrize("tx,ty,counts", [
+    (1, 1, [700]), (3, 2, [0, 63, 64, 65, 1, 128]), (5, 4, [1025, 0, 0, 0, 0, 2049, 4100]), (25, 21, [130, 0, 64, 700]),
+    (64, 32, [128, 0, 129, 1, 300]), (90, 60, [0, 40, 0, 1300])])
+def test_packed_slots_give_the_gradients_of_fixed_ones(cuda, tx, ty, counts):
+    """The list as long as its entries (the tiles' slots one after another) against the same list
+    with room for 4096 entries per tile (slots at fixed places); nothing is written past the
+    smaller buffer."""
+    T, w, h = tx * ty, 16 * tx - 3, 16 * ty - 5
+    rng = np.random.default_rng(T)
+    n, per = max(counts), np.resize(counts, T)
+    means = rng.uniform(-4.0, 20.0, (n, 2)) + 8.0 * np.array([tx, ty])
+    cov = np.zeros((n, 2, 2), F32)
+    s = max(w, h) * rng.uniform(0.3, 2.0, (n, 2))
+    cov[:, 0, 0], cov[:, 1, 1] = s[:, 0] ** 2, s[:, 1] ** 2
+    opac = (-5.5 + rng.normal(0, 0.3, (n, 1))).astype(F32)
+    col = rng.uniform(0, 1, (n, 3)).astype(F32)
+    rec = rasterizer.composite_records(*[torch.from_numpy(a).to(cuda) for a in (means.astype(F32), cov, opac, col)])
+    tiles = torch.from_numpy(np.repeat(np.arange(T), per).astype(np.int32)).to(cuda)
+    gids = torch.from_numpy(np.concatenate([np.arange(c) for c in per]).astype(np.int32)).to(cuda)
+    ranges = rasterizer.tile_ranges(tiles, T)
+    room = torch.zeros(4096 * T, dtype=torch.int32, device=cuda)
+    room[:gids.shape[0]] = gids
+    bg = torch.tensor([0.3, 0.1, 0.6], device=cuda)
+    cot = torch.from_numpy(rng.normal(0, 1, (h, w, 3)).astype(F32)).to(cuda)
+    out = []
+    for lst in (gids, room):
+        size = rasterizer.new_segments(h, w, cuda, lst.shape[0]).numel()
+        buf = torch.full((size + 65536,), 0xAB, dtype=torch.uint8, device=cuda)
+        segs = buf[:size]
+        image, fT, nc, _ = rasterizer.composite(rec, lst, ranges, h, w, bg, segments=segs)
+        grec, gbg = torch.empty((n, 12), device=cuda), torch.empty(3, device=cuda)
+        _lib.call("gs_composite_bwd_seg", _lib.stream_handle(cuda), n, _lib.ptr(rec), _lib.ptr(lst), lst.shape[0],
+                  _lib.ptr(ranges), w, h, _lib.ptr(bg), _lib.ptr(cot), None, None, None, _lib.ptr(fT), _lib.ptr(nc),
+                  _lib.ptr(segs), _lib.ptr(grec), _lib.ptr(gbg), 0, None, None)
+        assert bool((buf[size:] == 0xAB).all())
+        out.append((size, image, fT, nc, np_(grec), np_(gbg)))
+    (a, b) = out
+    assert a[0] < b[0] == rasterizer.new_segments(h, w, cuda).numel()
+    assert all(torch.equal(x, y) for x, y in zip(a[1:4], b[1:4]))
+    # the same terms, added by atomics in another order
+    assert rel(a[4], b[4]) <= 2e-5 and rel(a[5], b[5]) <= 1e-4
+
+
+def test_live_renders_of_a_small_scene_hold_little(cuda):
+    """Three renders of 2000 Gaussians at 1440x1079 before any backward: each holds its images, its
+    list (256 entries per Gaussian) and the segments of that many entries, not the 401 MB of lists of
+    4096 entries in every tile."""
+    sc = scenes.make_scene(1, n=2000, width=1440, height=1079)
+    g, cam, _, m = scenes.to_torch(sc, cuda)
+    g.means.requires_grad_(True)
+    held, live = [], []
+    for _ in range(3):
+        before = torch.cuda.memory_allocated()
+        live.append(render(g, cam, mask=m, sh_degree=sc["sh_degree"])[0])
+        held.append(torch.cuda.memory_allocated() - before)
+    assert max(held) < 100e6, held
+    sum(i.sum() for i in live).backward()
+    assert bool(torch.isfinite(g.means.grad).all())
