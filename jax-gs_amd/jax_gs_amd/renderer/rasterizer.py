@@ -175,6 +175,10 @@ def _composite_segments(records, sorted_gids, ranges, H, W, background, image, f
         _check_bins(bins, records, sorted_gids, ranges)
         stats, ws, capacity = bins["stats"], bins["workspace"], bins["capacity"]
         nb = ws.shape[0]
+    need = _lib.lib().gs_composite_segments_size_for(int(W), int(H), capacity)
+    if segments.device != dev or segments.numel() * segments.element_size() < need:
+        raise ValueError(f"composite: segments must hold {need} bytes on {dev} (new_segments(H, W, device, "
+                         f"{capacity}))")
     if l1_target is not None:
         tgt = check_f32("l1_target", l1_target, (H, W, 3), dev)
         l1_out = torch.empty((_lib.lib().gs_composite_l1_out_size(int(W), int(H)),), dtype=torch.float32, device=dev)

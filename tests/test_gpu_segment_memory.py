@@ -103,3 +103,20 @@ def test_live_renders_of_a_small_scene_hold_little(cuda):
     assert max(held) < 100e6, held
     sum(i.sum() for i in live).backward()
     assert bool(torch.isfinite(g.means.grad).all())
+
+
+def test_composite_refuses_segments_of_another_size(cuda):
+    """A buffer made for a smaller image or a shorter list, or on the host, is refused before the
+    launch that would write past it."""
+    w, h, n = 200, 120, 300
+    t, tiles, gids = _scene(cuda, n, w, h)
+    rec = rasterizer.composite_records(*t)
+    ranges = rasterizer.tile_ranges(tiles, ((w + 15) // 16) * ((h + 15) // 16))
+    bg = torch.zeros(3, device=cuda)
+    length = gids.shape[0]
+    good = rasterizer.new_segments(h, w, cuda, length)
+    for bad in (rasterizer.new_segments(h - 16, w, cuda, length), rasterizer.new_segments(h, w, cuda, 1000), good[:-256],
+                good.cpu()):
+        with pytest.raises(ValueError, match="segments must hold"):
+            rasterizer.composite(rec, gids, ranges, h, w, bg, segments=bad)
+    rasterizer.composite(rec, gids, ranges, h, w, bg, segments=good)
