@@ -552,7 +552,16 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
       Tend = te;
     }
   };
-  auto walk_pair = [&](const Step& k0, const Step& k1) {
+  auto add_colour = [&](float w, const Step& k) {
+    c0 = fmaf(w, k.b.z, c0);
+    c1 = fmaf(w, k.b.w, c1);
+    c2 = fmaf(w, k.c.x, c2);
+  };
+  // ODD: the batch holds a colour that is not finite, and the pixels that its entry does not reach
+  // must stay as they are (0 times it is not 0).  The walk of such a batch is a body of its own: a
+  // branch in the one body took 50k Gaussians at 640x479 from 53 to 56 us.
+  auto walk_pair = [&](auto odd_tag, const Step& k0, const Step& k1) {
+    constexpr bool ODD = decltype(odd_tag)::value;
     const float al0 = alpha(k0), al1 = alpha(k1);
     float ex0, all0, ex1, all1;
     products(al0, ex0, all0);
@@ -561,9 +570,8 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
     const float T2 = T1 * all1, b1 = T1 * ex1;
     const float w0 = b0 > kTMin ? al0 * b0 : 0.0f;  // rasterizer.py:206
     const float w1 = b1 > kTMin ? al1 * b1 : 0.0f;
-    c0 = fmaf(w1, k1.b.z, fmaf(w0, k0.b.z, c0));
-    c1 = fmaf(w1, k1.b.w, fmaf(w0, k0.b.w, c1));
-    c2 = fmaf(w1, k1.c.x, fmaf(w0, k0.c.x, c2));
+    if (!ODD || w0 != 0.0f) add_colour(w0, k0);
+    if (!ODD || w1 != 0.0f) add_colour(w1, k1);
     const uint64_t still = __ballot(T2 > kTMin);
     if (still != open) {
       close(k0, Tr, b0, T1);
@@ -594,23 +602,28 @@ __global__ __launch_bounds__(64) void composite_fwd_quad_kernel(
       seg_end = segment_start(seg + 1, sg.lu);
     }
     const int ns = stage_batch<7>(row, b0, lane, rx0, rx1, ry0, ry1, sa, sb, sc);
+    const bool odd = __ballot(!(fabsf(row.b.z) + fabsf(row.b.w) + fabsf(row.c.x) <= 3.402823466e38f)) != 0ull;
     row = load_row(rec, ahead_gid(g_ahead, num_g));
     g_ahead = probe_gid_ahead<WIN>(gids, start, b0 + 128 + lane, n, win, thr);
     if (ns == 0) continue;
     // steps in pairs (their exponents overlap), two sets of registers used in turn
-    Step x0 = read_step(0), x1 = read_step(4), y0, y1;
-    for (int s = 0;;) {
-      y0 = read_step(s + 8);
-      y1 = read_step(s + 12);
-      walk_pair(x0, x1);
-      s += 8;
-      if (s >= ns || open == 0ull) break;
-      x0 = read_step(s + 8);
-      x1 = read_step(s + 12);
-      walk_pair(y0, y1);
-      s += 8;
-      if (s >= ns || open == 0ull) break;
-    }
+    auto walk_steps = [&](auto odd_tag) {
+      Step x0 = read_step(0), x1 = read_step(4), y0, y1;
+      for (int s = 0;;) {
+        y0 = read_step(s + 8);
+        y1 = read_step(s + 12);
+        walk_pair(odd_tag, x0, x1);
+        s += 8;
+        if (s >= ns || open == 0ull) break;
+        x0 = read_step(s + 8);
+        x1 = read_step(s + 12);
+        walk_pair(odd_tag, y0, y1);
+        s += 8;
+        if (s >= ns || open == 0ull) break;
+      }
+    };
+    if (__builtin_expect(odd, 0)) walk_steps(BoolTag<true>{});
+    else walk_steps(BoolTag<false>{});
   }
   const bool closed = !((open >> lane) & 1ull);
   const float Tf = closed ? Tend : Tr;
@@ -1099,7 +1112,12 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
 // an rcp and a product.  Both NOCAP changes keep the loop-carried state in place (a body
 // chosen per entry between two versions made the compiler copy that state at every entry).
 // More registers live than the 64-VGPR build allows.
-template <int PPT, bool WIN, bool NOCAP, bool O32, bool SEG>
+// SEG: 0 walks whole lists, 1 and 2 the pieces of their segments.  2: a colour that is not finite
+// leaves the pixels that its entry does not reach as they are, as the one-pixel body (whose place
+// this one takes from kSegWideTiles tiles on) and the forward below kQuadTiles do; the others
+// evaluate pixel 0 with alpha 0, and 0 times such a colour is not 0.  A select per entry: 50k
+// Gaussians at 640x479 62.7 -> 63.3 us, so only there (2.1M at 1280x720 190.4 -> 192.6).
+template <int PPT, bool WIN, bool NOCAP, bool O32, int SEG>
 __device__ __forceinline__ void composite_bwd_body(
     const float4* __restrict__ rec, int num_g, const int32_t* __restrict__ gids, int64_t n_entries,
     const int32_t* __restrict__ ranges, int W, int H, int TX, int T, const float* __restrict__ bg,
@@ -1276,7 +1294,8 @@ __device__ __forceinline__ void composite_bwd_body(
               gc1 = fmaf(w, g1[i], gc1);
               gc2 = fmaf(w, g2[i], gc2);
               // c.g - Rg in one fma chain started from -Rg
-              const float dR = fmaf(e.b, g2[i], fmaf(e.g, g1[i], fmaf(e.r, g0[i], -Rg[i])));
+              float dR = fmaf(e.b, g2[i], fmaf(e.g, g1[i], fmaf(e.r, g0[i], -Rg[i])));
+              if (SEG == 2 && i == 0) dR = blends ? dR : 0.0f;
               const float dpw = w * dR;  // (alpha T) dR
               wdv[i] = dpw;
               Rg[i] = fmaf(al, dR, Rg[i]);
@@ -1433,7 +1452,7 @@ __device__ inline void clear_list_share(const ClearList& cl, int b, int nb, int 
 
 // What a workgroup walks: with segments (SEG), an item, none past their number; without, a
 // whole tile, from the launch order or the fixed one.
-template <bool SEG>
+template <int SEG>
 __device__ __forceinline__ bool walk_of_block(const Segments& sg, const int32_t* __restrict__ order, int TX, int T,
                                               int b, int& tile, int& piece) {
   if (SEG) {
@@ -1463,14 +1482,14 @@ __device__ __forceinline__ bool walk_of_block(const Segments& sg, const int32_t*
 // windows, as the forward read them.
 // Each workgroup zeroes its share of the clear list after its walk (stores issued before it
 // would hold up its first loads: loads and stores share one wait counter).
-template <bool WIN, bool O32, bool SEG>
+template <bool WIN, bool O32, int SEG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void composite_bwd_kernel(GS_BWD_PARAMS) {
   int tile, piece;
   if (walk_of_block<SEG>(sg, order, TX, T, blockIdx.x >> 2, tile, piece))
     composite_bwd_body<1, WIN, false, O32, SEG>(GS_BWD_ARGS, tile, piece, blockIdx.x & 3);
   clear_list_share(cl, blockIdx.x, gridDim.x, threadIdx.x);
 }
-template <bool WIN, bool O32, bool SEG>
+template <bool WIN, bool O32, int SEG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 5))) void composite_bwd_wide_kernel(
     GS_BWD_PARAMS) {
   int tile, piece;
@@ -1980,16 +1999,17 @@ int composite_bwd_run(const char* name, void* stream, int64_t n, const float* re
   // instructions per entry (1200 tiles: 66 us against 84 with four waves of one pixel per lane);
   // below, those four waves (24 tiles: 22 us against 40).
   const bool wide = segments ? T >= kSegWideTiles : pick_ppt(T) == 4;
-#define GS_BWD_LAUNCH1(WIN, O32, SEG)                                                                                \
-  if (wide) GS_BWD_LAUNCH((composite_bwd_wide_kernel<WIN, O32, SEG>), 1);                                            \
-  else GS_BWD_LAUNCH((composite_bwd_kernel<WIN, O32, SEG>), 4)
-#define GS_BWD_LAUNCH2(SEG)                                                                                          \
-  if (win && o32) { GS_BWD_LAUNCH1(true, true, SEG); }                                                               \
-  else if (o32) { GS_BWD_LAUNCH1(false, true, SEG); }                                                                \
-  else if (win) { GS_BWD_LAUNCH1(true, false, SEG); }                                                                \
-  else { GS_BWD_LAUNCH1(false, false, SEG); }
-  if (segments) { GS_BWD_LAUNCH2(true) } else { GS_BWD_LAUNCH2(false) }
-#undef GS_BWD_LAUNCH2
+#define GS_BWD_LAUNCH1(WIN, O32)                                                                                     \
+  if (!segments) {                                                                                                   \
+    if (wide) GS_BWD_LAUNCH((composite_bwd_wide_kernel<WIN, O32, 0>), 1);                                            \
+    else GS_BWD_LAUNCH((composite_bwd_kernel<WIN, O32, 0>), 4);                                                      \
+  } else if (T >= kQuadTiles) GS_BWD_LAUNCH((composite_bwd_wide_kernel<WIN, O32, 1>), 1);                            \
+  else if (wide) GS_BWD_LAUNCH((composite_bwd_wide_kernel<WIN, O32, 2>), 1);                                         \
+  else GS_BWD_LAUNCH((composite_bwd_kernel<WIN, O32, 2>), 4)
+  if (win && o32) { GS_BWD_LAUNCH1(true, true); }
+  else if (o32) { GS_BWD_LAUNCH1(false, true); }
+  else if (win) { GS_BWD_LAUNCH1(true, false); }
+  else { GS_BWD_LAUNCH1(false, false); }
 #undef GS_BWD_LAUNCH1
 #undef GS_BWD_LAUNCH
   GS_LAUNCH_CHECK("composite_bwd_kernel");
