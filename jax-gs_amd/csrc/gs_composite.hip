@@ -1115,8 +1115,8 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
 // SEG: 0 walks whole lists, 1 and 2 the pieces of their segments.  2: a colour that is not finite
 // leaves the pixels that its entry does not reach as they are, as the one-pixel body (whose place
 // this one takes from kSegWideTiles tiles on) and the forward below kQuadTiles do; the others
-// evaluate pixel 0 with alpha 0, and 0 times such a colour is not 0.  A select per entry: 50k
-// Gaussians at 640x479 62.7 -> 63.3 us, so only there (2.1M at 1280x720 190.4 -> 192.6).
+// evaluate pixel 0 with alpha 0, and 0 times such a colour is not 0.  A select per entry (50k
+// Gaussians at 640x479 62.6 -> 62.9 us), so only there.
 template <int PPT, bool WIN, bool NOCAP, bool O32, int SEG>
 __device__ __forceinline__ void composite_bwd_body(
     const float4* __restrict__ rec, int num_g, const int32_t* __restrict__ gids, int64_t n_entries,

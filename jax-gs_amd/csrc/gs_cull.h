@@ -16,13 +16,17 @@ __host__ __device__ inline float q_of(float dy, float Adx2l, float Bdx, float C)
   return fmaf(fmaf(C, dy, Bdx), dy, Adx2l);
 }
 
-__host__ __device__ inline float cull_rcp(float x) {
+// The cull's reciprocal: the hardware's on the device (1 ulp).  The CPU fuzz of the cull passes
+// reciprocals that are up to 2 ulp off in its place.
+struct CullRcp {
+  __host__ __device__ float operator()(float x) const {
 #ifdef __HIP_DEVICE_COMPILE__
-  return __builtin_amdgcn_rcpf(x);
+    return __builtin_amdgcn_rcpf(x);
 #else
-  return 1.0f / x;
+    return 1.0f / x;
 #endif
-}
+  }
+};
 
 // True when no point of the rectangle [x0,x1] x [y0,y1] can pass the gate
 // power > -10 for the entry (mx, my, A, B, C), where A dx^2 + B dx dy + C dy^2 =
@@ -41,13 +45,14 @@ __host__ __device__ inline float cull_rcp(float x) {
 // Every wave runs this for 64 entries at a time: two edges instead of four, no branches, no
 // division and no square root took the one-wave backward from 258 to 247 us (1M Gaussians,
 // 1920x1080).
+template <typename Rcp = CullRcp>
 __host__ __device__ inline bool entry_misses_rect(float mx, float my, float A, float B, float C, float x0,
-                                                  float x1, float y0, float y1) {
+                                                  float x1, float y0, float y1, Rcp rcp = Rcp()) {
   const float a = -A, b = -B, c = -C;
   const float dx0 = x0 - mx, dx1 = x1 - mx, dy0 = y0 - my, dy1 = y1 - my;
   const float nx = fminf(fmaxf(0.0f, dx0), dx1), ny = fminf(fmaxf(0.0f, dy0), dy1);
   // stationary points: dx* = sx dy, dy* = sy dx
-  const float sx = -0.5f * b * cull_rcp(a), sy = -0.5f * b * cull_rcp(c);
+  const float sx = -0.5f * b * rcp(a), sy = -0.5f * b * rcp(c);
   auto f = [&](float dx, float dy) { return fmaf(dx, fmaf(a, dx, b * dy), (c * dy) * dy); };
   const float fmin = fminf(f(nx, fminf(fmaxf(sy * nx, dy0), dy1)), f(fminf(fmaxf(sx * ny, dx0), dx1), ny));
   const float far_x = fmaxf(fabsf(dx0), fabsf(dx1)), far_y = fmaxf(fabsf(dy0), fabsf(dy1));

@@ -31,11 +31,12 @@ def fuzz_bin(tmp_path_factory):
 @pytest.mark.parametrize("seed", [1, 2])
 def test_no_false_drop_near_the_gate_boundary(fuzz_bin, seed):
     res = subprocess.run([fuzz_bin, "5000000", str(seed)], capture_output=True, text=True)
-    cases, dropped, false_drops, min_margin = res.stdout.split()
+    cases, dropped, false_drops, min_margin, dropped_4x4 = res.stdout.split()
     assert int(false_drops) == 0 and res.returncode == 0
     # the fuzz is not vacuous: a large share of the near-boundary cases is dropped, and the
     # closest dropped pixel sits just past the gate
     assert int(dropped) > int(cases) // 10
+    assert int(dropped_4x4) > int(cases) // 40  # of the quarter with the small images' 4x4 rectangles
     assert 0.0 <= float(min_margin) < 0.5
 
 
