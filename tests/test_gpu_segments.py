@@ -69,3 +69,40 @@ def test_segments_equal_whole_walks(cuda, tx, ty, counts, opacity, window):
     assert rel(out[1][0], out[0][0]) <= tol
     assert np.array_equal(out[1][0] == 0, out[0][0] == 0) or rel(out[1][0], out[0][0]) <= 1e-5
     assert rel(out[1][1], out[0][1]) <= 1e-4
+
+
+@pytest.mark.parametrize("w,h", [(128, 96), (504, 378), (1280, 720)])
+def test_segments_of_records_beyond_4gib(cuda, w, h):
+    """A walked record is addressed by its byte offset in a 32-bit register while the records span
+    less than 4 GiB, and by its id beyond: the same scene at the end of 4.3 GB of records, one
+    pixel per lane, four, and four from 2048 tiles on."""
+    from jax_gs_amd import scenes
+    from jax_gs_amd.renderer.projection import preprocess
+
+    sc = scenes.make_scene(2, n=20000, width=w, height=h)
+    g, cam, _, mask = scenes.to_torch(sc, cuda)
+    n_big = (2 ** 32 - 64) // (4 * _lib.GS_REC_STRIDE) + 1
+    with torch.no_grad():
+        pre = preprocess(g, cam, mask=mask, sh_degree=sc["sh_degree"])
+        b = rasterizer.bin_gaussians(pre["means2d"], pre["radii"], pre["valid"], pre["depths"], h, w,
+                                     want_tiles=False)
+    rec, gids, ranges = pre["records"], b["sorted_gids"], b["ranges"]
+    n = rec.shape[0]
+    big = torch.empty((n_big, _lib.GS_REC_STRIDE), device=cuda)
+    big[n_big - n:] = rec
+    bg = torch.tensor([0.1, 0.2, 0.3], device=cuda)
+    cot = torch.rand((h, w, 3), generator=torch.Generator(device=cuda).manual_seed(3), device=cuda)
+    images, grads = [], []
+    for rr, gg in ((rec, gids), (big, gids + (n_big - n))):
+        segs = rasterizer.new_segments(h, w, cuda, gg.shape[0])
+        image, fT, nc, _ = rasterizer.composite(rr, gg, ranges, h, w, bg, segments=segs)
+        grec = torch.empty_like(rr)
+        _lib.call("gs_composite_bwd_seg", _lib.stream_handle(cuda), rr.shape[0], _lib.ptr(rr), _lib.ptr(gg),
+                  gg.shape[0], _lib.ptr(ranges), w, h, _lib.ptr(bg), _lib.ptr(cot), None, None, None, _lib.ptr(fT),
+                  _lib.ptr(nc), _lib.ptr(segs), _lib.ptr(grec), None, 0, None, None)
+        images.append(image)
+        grads.append(np_(grec[-n:]))
+        assert not grec[:-n].any()
+    assert torch.equal(*images) and np.abs(grads[0]).max() > 0
+    # the same terms, added by atomics in another order
+    assert rel(grads[1], grads[0]) <= 1e-5
