@@ -14,9 +14,11 @@
 // Work decomposition: every wave owns PPT*4 rows of one 16x16 tile; lane l holds the
 // PPT pixels (l % 16, row0 + l / 16 + 4 i), i < PPT, i.e. one column, so the x offset
 // to a Gaussian is shared by the lane's pixels.  Waves are independent (no barriers).  With
-// PPT = 4 a wave covers the whole tile (used for large images); the backward of small images
-// takes PPT = 1 (four waves per tile), the forward of mid-size images PPT = 2 (two waves per
-// tile).  The forward of small images has a kernel of its own (composite_fwd_quad_kernel).
+// PPT = 4 a wave covers the whole tile: the forward from kFwdOneWaveTiles (6144) tiles on, the
+// backward of segments from kSegWideTiles (512), of whole lists from kQuadTiles (2048).  The
+// backward of fewer tiles takes PPT = 1 (four waves per tile), the forward of 2048 to 6143 tiles
+// PPT = 2 (two waves per tile).  The forward below 2048 tiles has a kernel of its own
+// (composite_fwd_quad_kernel).
 //
 // Culling: a Gaussian is binned to every tile its square 3-sigma box touches, but its
 // "power > -10" region is an ellipse, and for about a third of the (tile, entry) pairs
@@ -27,12 +29,13 @@
 // so an entry is dropped only if no pixel could pass the gate), and then walks the
 // surviving entries.  The walked entry is wave-uniform: its id comes from the
 // testing lane and its 48-byte record through scalar loads into SGPRs, prefetched
-// one surviving entry ahead.
+// one surviving entry ahead (the forward below 6144 tiles stages the survivors' records in LDS).
 //
-// Forward: branch-free per pixel; the wave stops when every pixel has T <= 1e-4
-// (ballot every 8 walked entries).  Per pixel it writes the final T and n_contrib,
+// Forward: branch-free per pixel; the wave stops when every pixel has T <= 1e-4 (tested every 8
+// walked entries, below 6144 tiles every 8 or 2).  Per pixel it writes the final T and n_contrib,
 // the number of leading entries met while T > 1e-4 (culled entries included).
-// Backward: replays each pixel back to front from (final T, n_contrib), recovering
+// Backward: replays each pixel back to front from (final T, n_contrib), or from the end of a
+// segment of the list (gs_segments.h), recovering
 // T_k = T_{k+1} / (1 - alpha_k) and the colour behind entry k projected on the
 // pixel's image cotangent g, Rg_{k-1} = alpha_k (c_k . g) + (1 - alpha_k) Rg_k, so
 // dL/dalpha_k = T_k (c_k . g - Rg_k).  Per lane the entry's power cotangents are kept
@@ -829,12 +832,10 @@ __global__ __launch_bounds__(64) void composite_fwd_kernel(
   auto walk = [&](uint64_t m, const int gk, auto kpos) __attribute__((always_inline)) {
     // The next survivor's record is requested before the current one is blended, into two
     // record registers used in turn, with an explicit wait before each request (scalar loads
-    // complete out of order: waiting for one is waiting for all; two-wave forward, cfg4
-    // 175 -> 155 us, cfg3 148 -> 135 us; one-wave cfg2 unchanged).
+    // complete out of order: waiting for one is waiting for all).
     // one walked entry e (tile index kidx within the batch) blended into the lane's pixels
-    // (two or four pixels per lane: branch-free, gated-out pixels blend alpha = 0, which
-    // leaves C and T unchanged; measured faster than per-pixel branches, 226 vs 251 us
-    // on cfg2)
+    // (branch-free, gated-out pixels blend alpha = 0, which leaves C and T unchanged; measured
+    // faster than per-pixel branches, 226 vs 251 us on cfg2)
     auto blend = [&](const Rec& e, int kidx) {
       const int kk = kpos(kidx) + 1;  // entries met so far, this one included
       const float dx = px - e.mx;
@@ -1467,8 +1468,8 @@ __device__ __forceinline__ bool walk_of_block(const Segments& sg, const int32_t*
   return tile >= 0 && tile < T;
 }
 
-// The backward's two builds.  One pixel per lane (images below 2048 tiles, four waves per
-// tile): 64 VGPRs, 8 waves per SIMD, the general body only (the no-cap path's per-entry test
+// The backward's two builds.  One pixel per lane (segments of images below kSegWideTiles tiles,
+// whole lists below kQuadTiles; four waves per tile or piece): 64 VGPRs, 8 waves per SIMD, the general body only (the no-cap path's per-entry test
 // costs more than it saves with one pixel per lane: cfg0 169 -> 174 us, cfg1 230 -> 236), four
 // walked entries per reduce-scatter (skipped when none of them blends a pixel of the wave):
 // cfg0 154 -> 142 us, cfg1 210 -> 199 against two.
@@ -1767,7 +1768,18 @@ inline bool rec_offsets_fit(int64_t n) { return n * (int64_t)(kRec * 4) <= (int6
 
 // Large images have enough tiles to fill the GPU with one wave per tile.
 inline int pick_ppt(int T) { return T >= kQuadTiles ? 4 : 1; }
+// Tiles from which a piece of a segmented list is walked by one wave of four pixels per lane, the
+// fewest instructions per entry, instead of four waves of one, the shortest chain.  Backward
+// launch with four waves -> one, 200k Gaussians in a uniform box: 256x256 (256 tiles) 45 -> 48 us,
+// 352x320 (440) 58 -> 53, 400x336 (525) 65 -> 55, 504x378 (768) 78 -> 62, 800x600 (1900) 145 -> 89;
+// 20k: 34 -> 50, 42 -> 46, 47 -> 46, 55 -> 51, 107 -> 66.  Where most entries lie in a few tiles the
+// chain counts for longer: 200k in 32 clusters 98 -> 184 at 256 tiles, 94 -> 177 at 525, 95 -> 158 at
+// 768, 117 -> 113 at 1200, 148 -> 120 at 1900 (20k: 31 -> 67, 32 -> 60, 36 -> 46, 47 -> 46, 62 -> 47).
+// The line is the even scene's; nothing the host knows tells the two apart.
 constexpr int kSegWideTiles = 512;
+static_assert(kSegWideTiles <= kQuadTiles, "from kQuadTiles tiles on pieces have the four-pixel build only");
+// composite_fwd_quad_kernel reads the entry list, which a deferred binning writes below these
+static_assert(kQuadTiles <= kDeferMinTiles, "the small images' forward needs the whole list");
 // Tiles from which the forward gives a tile one wave (four pixels per lane); below that (and
 // from 2048 tiles) two waves of eight rows each: at 3600 tiles a launch holds 3-4 waves per
 // SIMD, and halving the work units evens them out (cfg4 forward 189 -> 176 us) where at
@@ -1864,13 +1876,15 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
                      SB ? *sbl : none, gids_out, l1_target, l1_part, sg)
 #define GS_FWD_LAUNCH1(PPT, WPT, WIN, O32) \
   if (sbl) GS_FWD_LAUNCH2(PPT, WPT, WIN, O32, true); else GS_FWD_LAUNCH2(PPT, WPT, WIN, O32, false)
-#define GS_FWD_LAUNCH(PPT, WPT, WIN) \
-  if (o32) { GS_FWD_LAUNCH1(PPT, WPT, WIN, true); } else { GS_FWD_LAUNCH1(PPT, WPT, WIN, false); }
   const bool win = window != nullptr, o32 = rec_offsets_fit(n);
   if (pick_ppt(T) == 4 && T >= kFwdOneWaveTiles) {
-    if (win) { GS_FWD_LAUNCH(4, 1, true); } else { GS_FWD_LAUNCH(4, 1, false); }
+    if (win && o32) { GS_FWD_LAUNCH1(4, 1, true, true); }
+    else if (o32) { GS_FWD_LAUNCH1(4, 1, false, true); }
+    else if (win) { GS_FWD_LAUNCH1(4, 1, true, false); }
+    else { GS_FWD_LAUNCH1(4, 1, false, false); }
   } else if (pick_ppt(T) == 4) {
-    if (win) { GS_FWD_LAUNCH(2, 2, true); } else { GS_FWD_LAUNCH(2, 2, false); }
+    // every lane loads its own record: no offset register, one build for any number of records
+    if (win) { GS_FWD_LAUNCH1(2, 2, true, true); } else { GS_FWD_LAUNCH1(2, 2, false, true); }
   } else {
     // below kDeferMinTiles the entry list is always whole
 #define GS_FWD_QUAD(WIN)                                                                                          \
@@ -1881,7 +1895,6 @@ int composite_fwd_run(const char* name, void* stream, int64_t n, const float* re
     if (win) GS_FWD_QUAD(true); else GS_FWD_QUAD(false);
 #undef GS_FWD_QUAD
   }
-#undef GS_FWD_LAUNCH
 #undef GS_FWD_LAUNCH1
 #undef GS_FWD_LAUNCH2
   GS_LAUNCH_CHECK("composite_fwd_kernel");
@@ -1995,9 +2008,6 @@ int composite_bwd_run(const char* name, void* stream, int64_t n, const float* re
                      ranges, width, height, TX, T, background, gc, final_T, n_contrib, grad_records,                   \
                      tile_order, window, sg, cl)
   const bool win = window != nullptr, o32 = rec_offsets_fit(n);
-  // A piece is short: from 512 tiles on one wave of four pixels per lane walks it, the fewest
-  // instructions per entry (1200 tiles: 66 us against 84 with four waves of one pixel per lane);
-  // below, those four waves (24 tiles: 22 us against 40).
   const bool wide = segments ? T >= kSegWideTiles : pick_ppt(T) == 4;
 #define GS_BWD_LAUNCH1(WIN, O32)                                                                                     \
   if (!segments) {                                                                                                   \

@@ -110,8 +110,7 @@ __device__ inline float block_sum256(float v, float* red) {
 // the halo rows two vertically adjacent tiles share are fetched once.
 __device__ inline int ssim_tile_of_block(int b, int T) { return (b & 7) * ((T + 7) >> 3) + (b >> 3); }
 
-// Forward, CC channels (1..4), one channel at a time: the next channel's rows are loaded
-// into registers while the horizontal pass of the current one runs.
+// Forward, CC channels (1..4), one channel at a time.
 template <int CC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l1_ssim_fwd_kernel(
     int H, int W, int TX, int T, const float* __restrict__ x, const float* __restrict__ y, Taps taps,

@@ -13,7 +13,7 @@ gs_composite_fwd on the same inputs:
     over every pixel);
   * where the entry list must exist in full -- the default path's clamped chunk window, or
     more entries than the capacity -- the binning writes it all and the forward reads it.
-Cases: the compositing builds by tile count (four, two and one waves per tile), BASELINE
+Cases: the compositing builds by tile count (sixteen, two and one waves per tile), BASELINE
 configurations 2, 3 and 4 at full size (3: tiles beyond 4096 entries, the walk's cap),
 both rasterizer paths (window / own entries), Gaussians behind the camera, masked ones.
 """
@@ -49,7 +49,7 @@ def _prefix_positions(ranges, kmax):
 def _compare(sc, cuda, window, capacity=None, expect_deferred=True):
     c = sc["cam"]
     W, H = c["W"], c["H"]
-    # images under 2048 tiles (four waves per tile) get the whole list from the binning
+    # images under 2048 tiles (sixteen waves per tile) get the whole list from the binning
     expect_deferred = expect_deferred and ((W + 15) // 16) * ((H + 15) // 16) >= 2048
     g, cam, _, m = scenes.to_torch(sc, cuda)
     n = g.means.shape[0]

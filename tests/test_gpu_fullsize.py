@@ -3,12 +3,15 @@ picks (by tile count), and configurations 2, 3 and 4 of BASELINE.json at their
 configured sizes, against the CPU oracle (same bars as gpu_helpers.py).
 
 Kernel builds by tile count T (gs_composite.hip dispatch):
-  T < 2048          forward and backward with four waves per tile (one pixel per lane)
-  2048 <= T < 6144  two waves per tile forward (composite_fwd_kernel<2>), one wave per
-                    tile backward (composite_bwd_wide_kernel, with the path for entries
-                    no pixel of the wave sees at the 0.99 alpha cap)
-  T >= 6144         one wave per tile forward (composite_fwd_kernel<4>) and the same
-                    backward: the builds behind the headline numbers.
+  T < 2048          forward with sixteen waves of 4 x 4 pixels per tile
+                    (composite_fwd_quad_kernel); backward over the lists' segments, below
+                    512 tiles with four waves of one pixel per lane, else with one of four
+                    (composite_bwd_wide_kernel, with the path for entries no pixel of the
+                    wave sees at the 0.99 alpha cap)
+  2048 <= T < 6144  two waves per tile forward (composite_fwd_kernel<2>), the four-pixel
+                    backward over segments
+  T >= 6144         one wave per tile forward (composite_fwd_kernel<4>) and the four-pixel
+                    backward over whole lists: the builds behind the headline numbers.
 The dense scenes saturate many pixels (T <= 1e-4), so the wave-wide early exit, the
 per-pixel n_contrib < count and the backward's replay from saturated pixels are compared,
 not only the open-pixel paths.
