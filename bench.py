@@ -149,19 +149,21 @@ def main():
                                          want_tiles=False, window=True, deferred=True)
             mark("t2")
             grec = torch.empty((N, _lib.GS_REC_STRIDE), device=dev)  # cleared by the forward launch
-            # the compositing forward with the L1 loss fused (its partial sums, and the
-            # launch that orders the tiles for the backward finishes the loss)
-            image, fT, nc, order, loss = rasterizer.composite(pre["records"], b["sorted_gids"], b["ranges"], H, W,
-                                                              bg, clear_records=grec, window=b["window"], bins=b,
-                                                              l1_target=tgt)
+            # the compositing forward as the step runs it: the L1 loss fused (its partial sums; the
+            # launch that orders the backward's work finishes the loss), and below 6144 tiles
+            # the lists' segments left for the backward
+            segs = rasterizer.new_segments(H, W, dev, b["capacity"])
+            image, fT, nc, _, loss = rasterizer.composite(pre["records"], b["sorted_gids"], b["ranges"], H, W, bg,
+                                                          clear_records=grec, window=b["window"], bins=b,
+                                                          l1_target=tgt, segments=segs)
             mark("t3")
             # as in the step: the compositing VJP zeroes the five gradient arrays on the side
             # and the preprocessing VJP writes only the reached Gaussians' rows
             outs = [torch.empty_like(getattr(g, f)) for f in fields]
             cl = _lib.clear_list(*outs)
-            _lib.call("gs_composite_bwd_l1", s_, N, _lib.ptr(pre["records"]), _lib.ptr(b["sorted_gids"]),
+            _lib.call("gs_composite_bwd_seg", s_, N, _lib.ptr(pre["records"]), _lib.ptr(b["sorted_gids"]),
                       b["sorted_gids"].shape[0], _lib.ptr(b["ranges"]), W, H, _lib.ptr(bg), None, _lib.ptr(image),
-                      _lib.ptr(tgt), _lib.ptr(one), _lib.ptr(fT), _lib.ptr(nc), _lib.ptr(order), _lib.ptr(grec),
+                      _lib.ptr(tgt), _lib.ptr(one), _lib.ptr(fT), _lib.ptr(nc), _lib.ptr(segs), _lib.ptr(grec),
                       None, 1, _lib.ptr(b["window"]), ctypes.byref(cl))
             mark("t4")
             _lib.call("gs_preprocess_bwd", s_, N, g.sh_coeffs.shape[1], D, *[_lib.ptr(getattr(g, f).detach())
@@ -485,10 +487,9 @@ def measured_traffic(kernel, config):
 def measured_valu_busy(stage, config):
     """VALU-busy fraction of the stage's kernel from the committed SQ-counter summary of the
     same configuration, and that file; (None, None) when there is none."""
-    # the builds of the bench's launches (the forward's first template argument is the pixels
-    # per lane, which the image size picks): matched by prefix
-    kernels = {"composite_bwd": "composite_bwd_wide_kernel<true, true>",
-               "composite_fwd": "composite_fwd_kernel<"}
+    # the builds of the bench's launches (the image size picks them): matched by prefix
+    kernels = {"composite_bwd": ("composite_bwd_wide_kernel<true, true", "composite_bwd_kernel<true, true"),
+               "composite_fwd": ("composite_fwd_kernel<", "composite_fwd_quad_kernel<")}
     path = os.path.join(PROFILES, f"composite_valu_cfg{config}.md")
     if stage not in kernels or not os.path.exists(path):
         return None, None
