@@ -44,6 +44,11 @@ constexpr int kSRows = 4 + 2 * kSR;      // input rows of a thread's four output
 constexpr float kC1 = 0.01f * 0.01f;
 constexpr float kC2 = 0.03f * 0.03f;
 
+// A group of four values at any float: 16-byte accesses need only 4-byte alignment, so the rows of
+// images whose width is no multiple of four take them as well (value by value, four or twelve floats
+// apart from lane to lane, they took 979x546 x 3 from 20 to 23 us forward and 13.6 to 19 backward).
+typedef float f4any __attribute__((ext_vector_type(4), aligned(4)));
+
 struct Taps {
   float w[kSTaps];
 };
@@ -114,7 +119,7 @@ __device__ inline int ssim_tile_of_block(int b, int T) { return (b & 7) * ((T + 
 template <int CC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l1_ssim_fwd_kernel(
     int H, int W, int TX, int T, const float* __restrict__ x, const float* __restrict__ y, Taps taps,
-    float inv_count, float* __restrict__ gmap, bool vec, float2* __restrict__ partial) {
+    float inv_count, float* __restrict__ gmap, float2* __restrict__ partial) {
   __shared__ __align__(16) float V[5][kSTH][kSCols];
   __shared__ float red[4];
   const int tile = ssim_tile_of_block(blockIdx.x, T);
@@ -203,11 +208,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
       }
       if (gmap != nullptr) {
         float* __restrict__ g = gmap + (ch * H + orow) * W + ocol;
-        if (vec) {  // W a multiple of 4: whole groups, aligned
-          *reinterpret_cast<float4*>(g) = make_float4(G0[0], G0[1], G0[2], G0[3]);
-          *reinterpret_cast<float4*>(g + plane) = make_float4(G1[0], G1[1], G1[2], G1[3]);
-          *reinterpret_cast<float4*>(g + 2 * (int64_t)plane) = make_float4(G2[0], G2[1], G2[2], G2[3]);
-        } else {
+        if (ocol + 4 <= W) {
+          *reinterpret_cast<f4any*>(g) = f4any{G0[0], G0[1], G0[2], G0[3]};
+          *reinterpret_cast<f4any*>(g + plane) = f4any{G1[0], G1[1], G1[2], G1[3]};
+          *reinterpret_cast<f4any*>(g + 2 * (int64_t)plane) = f4any{G2[0], G2[1], G2[2], G2[3]};
+        } else {  // the row's last group
 #pragma unroll
           for (int o = 0; o < 4; ++o) {
             if (ocol + o >= W) break;
@@ -309,7 +314,7 @@ __device__ inline void loss_cot(const LossCot& c, float& g_l1, float& g_ss) {
 template <int CC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l1_ssim_bwd_kernel(
     int H, int W, int TX, int T, const float* __restrict__ x, const float* __restrict__ y, Taps taps,
-    float inv_count, const float* __restrict__ gmap, const LossCot cot, bool vec,
+    float inv_count, const float* __restrict__ gmap, const LossCot cot,
     float* __restrict__ grad) {
   __shared__ __align__(16) float V[3][kSTH][kSCols];
   const int tile = ssim_tile_of_block(blockIdx.x, T);
@@ -334,14 +339,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
 #pragma unroll
   for (int m = 0; m < 3; ++m) load_rows(gmap + m * plane, col, v[m]);
   float xq[4 * CC], yq[4 * CC];
-  if (vec) {
-    if (nval > 0) {
+  if (nval == 4 * CC) {
 #pragma unroll
-      for (int q = 0; q < CC; ++q) {
-        const float4 fx = reinterpret_cast<const float4*>(x + p)[q], fy = reinterpret_cast<const float4*>(y + p)[q];
-        xq[4 * q] = fx.x, xq[4 * q + 1] = fx.y, xq[4 * q + 2] = fx.z, xq[4 * q + 3] = fx.w;
-        yq[4 * q] = fy.x, yq[4 * q + 1] = fy.y, yq[4 * q + 2] = fy.z, yq[4 * q + 3] = fy.w;
-      }
+    for (int q = 0; q < CC; ++q) {
+      const f4any fx = reinterpret_cast<const f4any*>(x + p)[q], fy = reinterpret_cast<const f4any*>(y + p)[q];
+      xq[4 * q] = fx.x, xq[4 * q + 1] = fx.y, xq[4 * q + 2] = fx.z, xq[4 * q + 3] = fx.w;
+      yq[4 * q] = fy.x, yq[4 * q + 1] = fy.y, yq[4 * q + 2] = fy.z, yq[4 * q + 3] = fy.w;
     }
   } else {
 #pragma unroll
@@ -387,12 +390,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
       }
     }
   }
-  if (vec) {
-    if (nval > 0) {
+  if (nval == 4 * CC) {
 #pragma unroll
-      for (int q = 0; q < CC; ++q)
-        reinterpret_cast<float4*>(grad + p)[q] = make_float4(xq[4 * q], xq[4 * q + 1], xq[4 * q + 2], xq[4 * q + 3]);
-    }
+    for (int q = 0; q < CC; ++q)
+      reinterpret_cast<f4any*>(grad + p)[q] = f4any{xq[4 * q], xq[4 * q + 1], xq[4 * q + 2], xq[4 * q + 3]};
   } else {
 #pragma unroll
     for (int q = 0; q < 4 * CC; ++q)
@@ -583,11 +584,6 @@ struct SsimLayout {
   size_t gmap_off, part_off, total;
 };
 
-// Groups of four columns are whole and 16-byte aligned in arrays of this width.
-bool whole_groups(int width, const void* a, const void* b, const void* c) {
-  return width % 4 == 0 && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0;
-}
-
 SsimLayout ssim_layout(int H, int W, int C) {
   SsimLayout L;
   L.count = (int64_t)H * W * C;
@@ -626,13 +622,12 @@ int l1_ssim_fwd_run(const char* name, void* stream, int height, int width, int c
   const float inv = (float)(1.0 / (double)L.count);
   float2* part = (float2*)(ws + L.part_off);
   float* gmap = with_grad ? (float*)(ws + L.gmap_off) : nullptr;
-  const bool vec = whole_groups(width, gmap, nullptr, nullptr);
   const Taps taps = make_taps();
   switch (channels) {
-    case 1: hipLaunchKernelGGL(l1_ssim_fwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
-    case 2: hipLaunchKernelGGL(l1_ssim_fwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
-    case 3: hipLaunchKernelGGL(l1_ssim_fwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
-    default: hipLaunchKernelGGL(l1_ssim_fwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, vec, part); break;
+    case 1: hipLaunchKernelGGL(l1_ssim_fwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
+    case 2: hipLaunchKernelGGL(l1_ssim_fwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
+    case 3: hipLaunchKernelGGL(l1_ssim_fwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
+    default: hipLaunchKernelGGL(l1_ssim_fwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, part); break;
   }
   GS_LAUNCH_CHECK("l1_ssim_fwd_kernel");
   if (loss != nullptr)
@@ -676,13 +671,12 @@ int l1_ssim_bwd_run(const char* name, void* stream, int height, int width, int c
   hipStream_t s = (hipStream_t)stream;
   const float inv = (float)(1.0 / (double)L.count);
   const float* gmap = (const float*)((const char*)workspace + L.gmap_off);
-  const bool vec = whole_groups(width, pred, target, grad_pred);
   const Taps taps = make_taps();
   switch (channels) {
-    case 1: hipLaunchKernelGGL(l1_ssim_bwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
-    case 2: hipLaunchKernelGGL(l1_ssim_bwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
-    case 3: hipLaunchKernelGGL(l1_ssim_bwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
-    default: hipLaunchKernelGGL(l1_ssim_bwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, vec, grad_pred); break;
+    case 1: hipLaunchKernelGGL(l1_ssim_bwd_kernel<1>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, grad_pred); break;
+    case 2: hipLaunchKernelGGL(l1_ssim_bwd_kernel<2>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, grad_pred); break;
+    case 3: hipLaunchKernelGGL(l1_ssim_bwd_kernel<3>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, grad_pred); break;
+    default: hipLaunchKernelGGL(l1_ssim_bwd_kernel<4>, L.grid, dim3(256), 0, s, height, width, L.TX, L.T, pred, target, taps, inv, gmap, cot, grad_pred); break;
   }
   GS_LAUNCH_CHECK("l1_ssim_bwd_kernel");
   return GS_OK;

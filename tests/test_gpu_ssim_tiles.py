@@ -1,6 +1,6 @@
 """The L1 + SSIM kernels at the edges of their tiles (8 rows x 116 columns, groups of four columns
-that are stored whole where the width and the addresses allow it): means and image gradient
-against the float64 oracle."""
+that are read and stored whole at any address but for a row's last, shorter one): means and image
+gradient against the float64 oracle."""
 import numpy as np
 import pytest
 import torch
